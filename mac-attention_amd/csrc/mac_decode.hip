@@ -20,9 +20,10 @@
 //
 //  2. span_attention  (persistent grid sized to the device's residency)
 //     Every workgroup plans the same task list from the group spans: the long
-//     groups' spans are cut into chunks of C tokens (C picked from the total
-//     token count so that the grid gets ~12 tasks per workgroup; the last
-//     quarter of a long band in half chunks where the partial slots allow),
+//     groups' spans are cut into chunks of C tokens (C picked from their total
+//     token count so that the grid gets ~12 tasks per workgroup, or one each in
+//     a small step; the last quarter of a long band in half chunks where the
+//     partial slots allow),
 //     a short group left to this kernel is one task, and workgroups claim
 //     tasks through an atomic counter, full chunks first.  A task streams its
 //     K/V rows in 32-token blocks for all G query heads of the group (S^T =
@@ -1505,15 +1506,19 @@ __device__ __forceinline__ int group_chunk(int tokens, int chunk, int cap) {
 // group's pieces still fit `cap` partial slots; other bands are cut into full
 // chunks and one shorter remainder.  Span attention fetches the full pieces
 // first and the shorter ones after them, so the last tasks of a step are
-// short and the workgroups end close together.
+// short and the workgroups end close together.  Chunks below kTierMinChunk
+// are those of small steps cut evenly into one task per workgroup
+// (kSmallChunk): halving some of them would start a second round instead (2
+// x 64K, GQA-4, hit 0.5: 67 us of span attention tiered, 62 without).
 constexpr int kTierChunks = 4;
+constexpr int kTierMinChunk = 3072;
 
 __device__ __forceinline__ void band_layout(GroupSpans& s, int cap) {
   const int len = s.new_end - s.band_begin;
   s.n_full = len / s.chunk;
   s.piece2 = s.chunk;
   s.n_band = ceil_div(len, s.chunk);
-  if (s.n_full >= kTierChunks) {
+  if (s.n_full >= kTierChunks && s.chunk >= kTierMinChunk) {
     const int half = ((s.chunk >> 1) + 63) & ~63;
     const int f = (len - len / 4) / s.chunk;
     const int n = f + ceil_div(len - f * s.chunk, half);
@@ -1586,14 +1591,23 @@ __device__ __forceinline__ int block_exclusive_scan(int v, int* s_tmp, int& tota
 // while a task of at least kMinChunk tokens amortises its fixed cost (plan
 // lookup, Q staging, pipeline fill, partial write) and keeps a long group's
 // partials few enough for merge_write to fetch in one or two rounds.
+// A step too small for one such task per workgroup (fewer than kMinChunk
+// tokens each) is cut evenly into one task per workgroup, down to
+// kSmallChunk tokens (two blocks per wave, about a task's fixed cost): with
+// kMinChunk-token tasks most CUs had none, and the few tasks were serial
+// chains.  Span attention (us), kMinChunk tasks / one per workgroup / two:
+// 1 x 4K GQA-4 hit 0.5 61 / 26 / 26; 1 x 32K the same 65 / 35 / 40; 1 x 127K
+// GQA-8 hit 0 88 / 60 / 59; 16 ragged contexts to 16K, hit 0.9, 63 / 34 / 35.
 constexpr int kTasksPerWorkgroup = 12;  // default of AttnParams::tasks_per_wg
 constexpr int kMinChunk = 3072;
+constexpr int kSmallChunk = 256;
 constexpr int kMaxChunk = 16384;
 constexpr int kFuseTokens = 1024;  // default of DecideParams::fuse_tokens
 
 // Every workgroup of span_attention derives the same task list: the chunk C
-// from the total token count of all groups (kTasksPerWorkgroup tasks per
-// workgroup, a multiple of 64 tokens in [kMinChunk, kMaxChunk]), then the
+// from the total token count of the long groups (kTasksPerWorkgroup tasks per
+// workgroup, a multiple of 64 tokens in [kMinChunk, kMaxChunk]; less for small
+// steps, see kSmallChunk), then the
 // tasks in two classes, largest first: class A holds the band pieces of full
 // chunk length, class B everything shorter (sinks, band remainders, tails,
 // and the whole bands of hit groups).  Workgroups fetch A tasks before B
@@ -1624,27 +1638,34 @@ __device__ void plan_tasks(const AttnParams& p, int* s_off, int* s_tmp, int& tot
     active_wgs_out = 0;
     return;
   }
+  // tok: tokens of the groups longer than fuse_tokens, which the chunk and
+  // the grid follow from (a short group is one task wherever it runs, and
+  // where it runs depends on earlier steps: counted here, it would make the
+  // cut of the long groups, and so their rounding, depend on them too);
+  // n_here: groups left to this kernel
   long long tok = 0;
+  int n_here = 0;
   for (int g = g_lo; any_long && g < g_hi; ++g) {  // (all four loads in one round)
     const int fused = p.group_fused[g];  // finished by match_decide
     const int ne = p.group_rect_end[g];
     const int t = group_tokens(min(p.F, ne), p.group_rect_begin[g], ne, p.group_tail_end[g]);
-    tok += fused != 0 ? 0 : t;
+    tok += (p.fuse_tokens > 0 && t <= p.fuse_tokens) ? 0 : t;
+    n_here += fused != 0 ? 0 : 1;
   }
-  // reduce token count (64-bit) across the block
+  // reduce both across the block
   if (any_long) {
     long long x = tok;
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) x += __shfl_xor(x, off);
     __shared__ long long s_tok[kWaves];
     if (lane == 0) s_tok[wave] = x;
-    __syncthreads();
+    n_here = __syncthreads_or(n_here);
     tok = 0;
 #pragma unroll
     for (int w = 0; w < kWaves; ++w) tok += s_tok[w];
     __syncthreads();
   }
-  if (tok == 0 && blockIdx.x != 0) {  // nothing to attend: only workgroup 0 publishes the counters
+  if (n_here == 0 && blockIdx.x != 0) {  // nothing to attend: only workgroup 0 publishes the counters
     total_tasks_out = 0;
     chunk_out = 0;
     active_wgs_out = 0;
@@ -1657,9 +1678,10 @@ __device__ void plan_tasks(const AttnParams& p, int* s_off, int* s_tmp, int& tot
   active_wgs_out = W;
   const long long target_tasks = static_cast<long long>(p.tasks_per_wg) * W;
   int chunk = static_cast<int>((tok + target_tasks - 1) / target_tasks);
-  chunk = ceil_div(max(chunk, p.min_chunk), 64) * 64;
+  const int even = static_cast<int>(min((tok + W - 1) / W, static_cast<long long>(p.min_chunk)));
+  chunk = ceil_div(max(chunk, max(even, kSmallChunk)), 64) * 64;
   chunk = min(chunk, kMaxChunk);
-  if (tok == 0) {  // nothing to attend (only workgroup 0 is here): publish an empty plan
+  if (n_here == 0) {  // nothing to attend (only workgroup 0 is here): publish an empty plan
     if (tid == 0) {
       p.task_counts[0] = 0;
       p.task_counts[4] = chunk;
@@ -1673,7 +1695,7 @@ __device__ void plan_tasks(const AttnParams& p, int* s_off, int* s_tmp, int& tot
   // bucket unless the batch has more groups than the table has entries).
   int* s_offb = s_off + NB + 1;
   int my_a = 0, my_b = 0;
-  for (int g = g_lo; tok > 0 && g < g_hi; ++g) {
+  for (int g = g_lo; g < g_hi; ++g) {
     GroupSpans sp = load_spans(p.group_rect_begin, p.group_rect_end, p.group_tail_end, g, p.F, chunk, p.cap);
     int na, nb;
     group_task_counts(sp, p.group_fused[g] != 0, p.fuse_tokens, na, nb);
@@ -1690,7 +1712,7 @@ __device__ void plan_tasks(const AttnParams& p, int* s_off, int* s_tmp, int& tot
   int total_a = 0, total_b = 0;
   int base_a = block_exclusive_scan(my_a, s_tmp, total_a);
   int base_b = block_exclusive_scan(my_b, s_tmp, total_b);
-  for (int b = g_lo / gpb; tok > 0 && b * gpb < g_hi; ++b) {
+  for (int b = g_lo / gpb; b * gpb < g_hi; ++b) {
     const int ca = s_off[b], cb = s_offb[b];
     s_off[b] = base_a;
     s_offb[b] = total_a + base_b;

@@ -441,3 +441,34 @@ def test_step_fuse_rule(case, ext, monkeypatch):
         assert go[2 * ng + 2:2 * ng + 4].tolist() == [ng - long_groups, long_groups]
         assert go[2 * ng + 4] == sum(-(-t // 64) for t in _group_tokens(c))
         prev = ws[16].clone()
+
+
+@pytest.mark.parametrize("hkv,kv_lens,fuse", [
+    (8, [1100], "auto"),          # just past a short group: the smallest chunk
+    (4, [33, 2000, 1025], "split"),  # pieces of a block and less beside full chunks
+    (8, [40000, 9, 17000, 1300], "auto"),  # cut evenly, between the smallest and the multi-round chunk
+    (1, [130000], "auto"),        # one group, every task its own workgroup
+])
+def test_small_step_chunks(hkv, kv_lens, fuse, ext, monkeypatch):
+    """The chunk of a step too small for one multi-round chunk per workgroup:
+    the long groups' tokens spread evenly over the grid, a multiple of 64 in
+    [256, 3072], the same wherever the short groups ran; results against the
+    oracle."""
+    _set_fuse(monkeypatch, fuse)
+    print(f"small step: hkv={hkv} kv_lens={kv_lens} {fuse}", flush=True)
+    c = syn.random_case(batch=len(kv_lens), hq=4 * hkv, hkv=hkv, kv_lens=kv_lens, capacity=32, semantic_pos_ahead=64,
+                        front_sink_tokens=16, hit_rate=0.0, seed=7)
+    ws = syn.workspace(torch, batch=len(kv_lens), hq=4 * hkv, hkv=hkv, capacity=32, max_context=131072, tile_tokens=32,
+                       match_tile_slots=8, semantic_pos_ahead=64, front_sink_tokens=16, device="cuda")
+    ws[16].zero_()
+    res = oracle_run(c)
+    grid = 2 * torch.cuda.get_device_properties(0).multi_processor_count
+    short = 0 if fuse == "split" else 1024
+    tokens = sum(hkv * kv for kv in kv_lens if kv > short)
+    chunk = -(-max(min(-(-tokens // grid), 3072), 256, -(-tokens // (12 * grid))) // 64) * 64
+    for step in ("first", "repeat"):  # (the second finds the first's counts)
+        dev = syn.to_device(torch, c)
+        out, out_lse, w = syn.run_decode(torch, ext, dev, c, max_context=131072, tile_tokens=32, match_tile_slots=8, ws=ws)
+        torch.cuda.synchronize()
+        assert int(_np(w[22])[4]) == chunk, step
+        _check_against_oracle(c, dev, out, out_lse, w, res, what=f"small step {step}")
