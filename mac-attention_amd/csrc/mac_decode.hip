@@ -1944,14 +1944,20 @@ __global__ void __launch_bounds__(kBlock, 2) span_attention_mfma_kernel(AttnPara
 
 // ============================================================ 3. merge ====
 
-// One workgroup per (group, query head); lane l of every wave owns dims
-// 2l, 2l+1.  The partials are split over the four waves (eight loads in
-// flight at a time) and loaded in one pass, so a full-fallback group with
-// hundreds of partials is merged in a fraction of the serial latency; the
-// four wave states are combined through LDS.  Per head (DECODE:4280-4685):
-// ring state = cached entry (hit heads) (+) band partials -> ring row (ready
-// requests only); out / out_lse = ring state (+) sink and tail partials.  An empty partial (lse = -inf) has weight 0,
-// the reference's skip rule (DECODE:866-890).
+// One workgroup per (group, query head).  The partials are dealt to the four
+// waves; a wave computes the weights of up to 64 of them at once, one per
+// lane, and then sums their rows (16-byte loads, two rows per instruction,
+// eight loads in flight behind the eight being summed); the four wave states
+// are combined through LDS.  Latency-bound: a chain of load rounds.  Merging
+// the rows one after the other put an exponential, a logarithm and a division
+// between every two of them and moved 8 bytes per load: 12.7 us against 8.9 for
+// 128 partials per head, 20 against 15 for 155 (with the kernel's events).  16
+// waves per head were slower below about 100 partials (9.9 for the 128) and at
+// every larger grid (20 against 9 at 64 groups x 8 heads).  Per head
+// (DECODE:4280-4685): ring state = cached entry (hit heads) (+) band partials
+// -> ring row (ready requests only); out / out_lse = ring state (+) sink and
+// tail partials.  An empty partial (lse = -inf) has weight 0, the reference's
+// skip rule (DECODE:866-890).
 // The per-group descriptors (chunk, task, band and tail task counts) and the
 // reference's task counters of the step (DECODE:1406-1530), counted by one
 // extra workgroup of merge_write, where they overlap that launch instead of
@@ -2045,7 +2051,8 @@ __device__ void publish_counts(const MergeParams& p) {
 // workgroups of blockIdx.x = 0 count (publish_counts, y = 0) or return.
 template <int G>
 __global__ void __launch_bounds__(kBlock) merge_write_kernel(MergeParams p) {
-  constexpr int kBatch = 8;
+  constexpr int kBatch = 8;  // 16-byte loads in flight per lane
+  constexpr int W = kWaves;
   if (blockIdx.x == 0) {
     if (blockIdx.y == 0) publish_counts(p);
     return;
@@ -2097,28 +2104,9 @@ __global__ void __launch_bounds__(kBlock) merge_write_kernel(MergeParams p) {
   band_layout(sp, p.cap);
   const int n_sink = sp.n_sink, n_band = sp.n_band, n_tail = sp.n_tail;
 
-  __shared__ float s_o[2][kWaves][kHeadDim];
-  __shared__ float s_l[2][kWaves];
+  __shared__ __align__(16) float s_o[2][W][kHeadDim];
+  __shared__ float s_m[2][W], s_l[2][W];
 
-  auto load_partial = [&](int j, float& lse2, float& o0, float& o1) {
-    const int64_t slot = static_cast<int64_t>(g) * p.cap + j;
-    lse2 = p.partial_lse[slot * G + h];
-    const int64_t oi = static_cast<int64_t>(g) * p.o_group_stride + (static_cast<int64_t>(j) * G + h) * kHeadDim + d0;
-    if (p.partial_bf16) {
-      const uint32_t w = *reinterpret_cast<const uint32_t*>(static_cast<const uint16_t*>(p.partial_o) + oi);
-      o0 = bf16_lo(w);
-      o1 = bf16_hi(w);
-    } else {
-      const float2 v = *reinterpret_cast<const float2*>(static_cast<const float*>(p.partial_o) + oi);
-      o0 = v.x;
-      o1 = v.y;
-    }
-  };
-
-  // One pass over all partials of the group (wave w takes j = w, w + 4, ...,
-  // eight loads in flight at a time): band partials into `ring` (on top of
-  // the cached entry), sink and tail partials into `rest`.
-  MergeState ring{-INFINITY, {0.0f, 0.0f}}, rest{-INFINITY, {0.0f, 0.0f}};
   // The cached entry of a hit head (wave 0): its lse and o are loaded
   // together here and merged after the partials, so the partial loads are
   // issued without waiting for them.  A non-finite lse is skipped.
@@ -2129,43 +2117,120 @@ __global__ void __launch_bounds__(kBlock) merge_write_kernel(MergeParams p) {
     entry_lse = p.lse_cache[rowi];
     entry_o = *reinterpret_cast<const uint32_t*>(p.attn_cache + rowi * kHeadDim + d0);
   }
-  // this wave's partials of [j0, j1) into `st`, eight loads in flight; wave
-  // (first + k) % 4 takes j0 + k, so that consecutive ranges continue the
-  // rotation instead of all starting on wave 0
-  auto merge_range = [&](MergeState& st, int j0, int j1, int first) {
-    for (int jb = j0 + ((wave - first) & (kWaves - 1)); jb < j1; jb += kWaves * kBatch) {
-      float pl[kBatch], p0[kBatch], p1[kBatch];
+
+  // One pass over the group's pieces in slot order (sink, band, tail; piece
+  // j to wave j % W), up to 64 per wave at a time: lane u holds the lse of
+  // the wave's piece u, so the weights of all of them take one exponential
+  // per lane, and the rows are then summed with no chain of exponentials and
+  // logarithms between them.  A lane takes four dims of every second piece
+  // (16-byte loads, two rows per instruction), kBatch loads in flight while
+  // the batch before them is summed.  Band pieces go to the ring class (c =
+  // 0), the others to the rest (c = 1): weights relative to the class's
+  // running maximum m, sums l and o.
+  const int np = n_sink + n_band + n_tail;
+  const int band_end = n_sink + n_band;
+  const int mine = np > wave ? (np - wave + W - 1) / W : 0;  // pieces of this wave
+  const int half = lane >> 5, dq = 4 * (lane & 31);
+  float m_c[2] = {kNegBig, kNegBig}, l_c[2] = {0.0f, 0.0f};
+  f32x4_t o_c[2] = {{0.0f, 0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f, 0.0f}};
+  auto load_row = [&](int u) -> f32x4_t {  // dims dq .. dq + 3 of the wave's piece u (clamped)
+    const int j = min(u, mine - 1) * W + wave;
+    const int64_t oi = static_cast<int64_t>(g) * p.o_group_stride + (static_cast<int64_t>(j) * G + h) * kHeadDim + dq;
+    if (p.partial_bf16) {
+      const uint2 w = *reinterpret_cast<const uint2*>(static_cast<const uint16_t*>(p.partial_o) + oi);
+      return f32x4_t{bf16_lo(w.x), bf16_hi(w.x), bf16_lo(w.y), bf16_hi(w.y)};
+    }
+    const float2* v = reinterpret_cast<const float2*>(static_cast<const float*>(p.partial_o) + oi);
+    return f32x4_t{v[0].x, v[0].y, v[1].x, v[1].y};
+  };
+  for (int u0 = 0; u0 < mine; u0 += 64) {
+    const int j = (u0 + lane) * W + wave;
+    float lse = -INFINITY;
+    if (u0 + lane < mine) lse = p.partial_lse[(static_cast<int64_t>(g) * p.cap + j) * G + h];
+    const int n = min(64, mine - u0);
+    f32x4_t a[kBatch];
 #pragma unroll
-      for (int u = 0; u < kBatch; ++u) {
-        const int j = jb + kWaves * u;
-        load_partial(j < j1 ? j : j0, pl[u], p0[u], p1[u]);
-        if (j >= j1) pl[u] = -INFINITY;
+    for (int u = 0; u < kBatch; ++u) a[u] = load_row(u0 + 2 * u + half);
+    const bool some = isfinite(lse);  // an empty piece has weight 0 (DECODE:866-890)
+    const bool band = j >= n_sink && j < band_end;
+    const float x = some ? lse * kLog2e : kNegBig;
+    float weight = 0.0f;
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+      const bool in_c = some && band == (c == 0);
+      float mx = in_c ? x : kNegBig;
+#pragma unroll
+      for (int off = 1; off < 64; off <<= 1) mx = fmaxf(mx, __shfl_xor(mx, off));
+      mx = fmaxf(mx, m_c[c]);
+      const float keep = fast_exp2(m_c[c] - mx);
+      m_c[c] = mx;
+      const float w = in_c ? fast_exp2(x - mx) : 0.0f;
+      float sum = w;
+#pragma unroll
+      for (int off = 1; off < 64; off <<= 1) sum += __shfl_xor(sum, off);
+      l_c[c] = l_c[c] * keep + sum;
+      o_c[c] *= keep;
+      if (in_c) weight = w;
+    }
+    for (int ub = 0; ub < n; ub += 2 * kBatch) {
+      f32x4_t b[kBatch];
+      if (ub + 2 * kBatch < n) {
+#pragma unroll
+        for (int u = 0; u < kBatch; ++u) b[u] = load_row(u0 + ub + 2 * (kBatch + u) + half);
       }
 #pragma unroll
-      for (int u = 0; u < kBatch; ++u) merge_into(st, pl[u], p0[u], p1[u]);
+      for (int u = 0; u < kBatch; ++u) {
+        const int k = ub + 2 * u + half;
+        const float w = __shfl(weight, min(k, 63));  // (0 past the wave's last piece)
+        const int ju = (u0 + k) * W + wave;
+        const bool in_ring = ju >= n_sink && ju < band_end;
+        // (an empty piece's row is not used: it may hold anything)
+        const bool used = k < n && w != 0.0f;
+        const f32x4_t y = used ? w * a[u] : f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          o_c[0][i] += in_ring ? y[i] : 0.0f;
+          o_c[1][i] += in_ring ? 0.0f : y[i];
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < kBatch; ++u) a[u] = b[u];
     }
-  };
-  merge_range(ring, n_sink, n_sink + n_band, 0);
-  merge_range(rest, n_sink + n_band, n_sink + n_band + n_tail, n_band);
-  merge_range(rest, 0, n_sink, n_band + n_tail);
-  merge_into(ring, entry_lse, bf16_lo(entry_o), bf16_hi(entry_o));
-  // the four waves' states, combined by wave 0 (which also read the entry:
-  // the entry read precedes the ring write below in the same lanes)
-  s_o[0][wave][d0] = ring.o[0];
-  s_o[0][wave][d0 + 1] = ring.o[1];
-  s_o[1][wave][d0] = rest.o[0];
-  s_o[1][wave][d0 + 1] = rest.o[1];
-  if (lane == 0) {
-    s_l[0][wave] = ring.lse;
-    s_l[1][wave] = rest.lse;
+  }
+  // the waves' states, combined by wave 0 (which also read the entry: the
+  // entry read precedes the ring write below in the same lanes)
+#pragma unroll
+  for (int c = 0; c < 2; ++c) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) o_c[c][i] += __shfl_xor(o_c[c][i], 32);
+    if (half == 0) *reinterpret_cast<f32x4_t*>(&s_o[c][wave][dq]) = o_c[c];
+    if (lane == 0) {
+      s_m[c][wave] = m_c[c];
+      s_l[c][wave] = l_c[c];
+    }
   }
   __syncthreads();
   if (wave != 0) return;
+  MergeState st[2];
 #pragma unroll
-  for (int w = 1; w < kWaves; ++w) {
-    merge_into(ring, s_l[0][w], s_o[0][w][d0], s_o[0][w][d0 + 1]);
-    merge_into(rest, s_l[1][w], s_o[1][w][d0], s_o[1][w][d0 + 1]);
+  for (int c = 0; c < 2; ++c) {
+    float mx = kNegBig, l = 0.0f, o0 = 0.0f, o1 = 0.0f;
+#pragma unroll
+    for (int w = 0; w < W; ++w) mx = fmaxf(mx, s_m[c][w]);
+#pragma unroll
+    for (int w = 0; w < W; ++w) {
+      const float f = fast_exp2(s_m[c][w] - mx);
+      l += s_l[c][w] * f;
+      o0 += s_o[c][w][d0] * f;
+      o1 += s_o[c][w][d0 + 1] * f;
+    }
+    const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+    st[c].lse = l > 0.0f ? (mx + fast_log2(l)) * kLn2 : -INFINITY;
+    st[c].o[0] = o0 * inv;
+    st[c].o[1] = o1 * inv;
   }
+  MergeState ring = st[0], rest = st[1];
+  merge_into(ring, entry_lse, bf16_lo(entry_o), bf16_hi(entry_o));
 
   if (ready && P >= 0) {  // ring row at past_len % M (a negative past_len has no ring slot)
     const int64_t rowi = (static_cast<int64_t>(req) * M + dest) * Hq + hq;

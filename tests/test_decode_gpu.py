@@ -447,9 +447,11 @@ def test_step_fuse_rule(case, ext, monkeypatch):
     (8, [1100], "auto"),          # just past a short group: the smallest chunk
     (4, [33, 2000, 1025], "split"),  # pieces of a block and less beside full chunks
     (8, [40000, 9, 17000, 1300], "auto"),  # cut evenly, between the smallest and the multi-round chunk
-    (1, [130000], "auto"),        # one group, every task its own workgroup
+    (1, [130000], "auto"),        # one group, every task its own workgroup: 500 partials per head to merge
+    (1, [130000, 5000, 41000], "auto"),
 ])
-def test_small_step_chunks(hkv, kv_lens, fuse, ext, monkeypatch):
+@pytest.mark.parametrize("partial", ["f32", "bf16"])
+def test_small_step_chunks(partial, hkv, kv_lens, fuse, ext, monkeypatch):
     """The chunk of a step too small for one multi-round chunk per workgroup:
     the long groups' tokens spread evenly over the grid, a multiple of 64 in
     [256, 3072], the same wherever the short groups ran; results against the
@@ -459,7 +461,8 @@ def test_small_step_chunks(hkv, kv_lens, fuse, ext, monkeypatch):
     c = syn.random_case(batch=len(kv_lens), hq=4 * hkv, hkv=hkv, kv_lens=kv_lens, capacity=32, semantic_pos_ahead=64,
                         front_sink_tokens=16, hit_rate=0.0, seed=7)
     ws = syn.workspace(torch, batch=len(kv_lens), hq=4 * hkv, hkv=hkv, capacity=32, max_context=131072, tile_tokens=32,
-                       match_tile_slots=8, semantic_pos_ahead=64, front_sink_tokens=16, device="cuda")
+                       match_tile_slots=8, semantic_pos_ahead=64, front_sink_tokens=16, device="cuda",
+                       partial_dtype=torch.float32 if partial == "f32" else torch.bfloat16)
     ws[16].zero_()
     res = oracle_run(c)
     grid = 2 * torch.cuda.get_device_properties(0).multi_processor_count
