@@ -1738,18 +1738,21 @@ __device__ void plan_tasks(const AttnParams& p, int* s_off, int* s_tmp, int& tot
   chunk_out = chunk;
 }
 
-// Dynamic task fetch: the counter is zeroed by match_decide, which runs
-// before this kernel on the same stream, so every step (and every graph
-// replay) starts from task 0.  Ends with a barrier, so the previous task's
-// LDS use is complete before the caller starts the next one.  (Claiming the
+// Dynamic task fetch after a workgroup's first task (its own index: no
+// claim, so the grid does not queue up on one counter as it starts, and a
+// step of at most one task per workgroup never touches it): the counter is
+// zeroed by match_decide, which runs before this kernel on the same stream,
+// so every step (and every graph replay) starts from 0.  Ends with a barrier,
+// so the previous task's LDS use is complete before the caller starts the
+// next one.  (Claiming the
 // next task one task ahead hides the atomic's round trip but hands two tasks
 // to the first workgroups when there are about as many tasks as workgroups,
 // which measured slower.)
-__device__ __forceinline__ int next_task(const AttnParams& p, int& s_task) {
+__device__ __forceinline__ int next_task(const AttnParams& p, int active_wgs, int& s_task) {
   __syncthreads();
   if (threadIdx.x == 0) s_task = atomicAdd(p.task_counter, 1);
   __syncthreads();
-  return s_task;
+  return active_wgs + s_task;
 }
 
 struct TaskInfo {
@@ -1933,12 +1936,13 @@ __global__ void __launch_bounds__(kBlock, 2) span_attention_mfma_kernel(AttnPara
   if (static_cast<int>(blockIdx.x) >= active_wgs || total_tasks == 0) return;
 
   __shared__ int s_task;
-  for (int t = next_task(p, s_task); t < total_tasks; t = next_task(p, s_task)) {
+  for (int t = blockIdx.x; t < total_tasks; t = next_task(p, active_wgs, s_task)) {
     const TaskInfo ti = decode_task(p, s_off, NG, chunk, t);
     if (ti.shrt)
       short_task<G>(p, ti, &s_kv[0][0][0], s_q, &s_ml[0][0][0][0], s_rect, s_mslot, s_entry);
     else
       mfma_task<G>(p, ti, s_kv, s_q, s_ml[0]);
+    if (total_tasks <= active_wgs) return;
   }
 }
 
