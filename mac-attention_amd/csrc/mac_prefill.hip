@@ -10,9 +10,9 @@
 //
 //  * downdate_kernel: the reference's downdate op on its own (any head_dim,
 //    f32/bf16/f16 lse), for callers that keep the reference's three calls.
-//  * window_kernel<HPW, false>: causal sliding-window attention over a
+//  * window_kernel<RT, kPlain>: causal sliding-window attention over a
 //    ragged batch with a page-size-1 KV pool (the windowed FlashInfer pass).
-//  * window_kernel<HPW, true>: the fused form.  Only the rows the ring keeps
+//  * window_kernel<RT, kRectify>: the fused form.  Only the rows the ring keeps
 //    (the last min(len, M) of each request) are computed; for them the window
 //    state never leaves registers: it is downdated from the full state and
 //    stored straight into the ring with the pre-RoPE query, followed by the
@@ -21,10 +21,10 @@
 // Both forms run S^T[key][row] = K Q^T and O^T[d][row] += V^T P^T on
 // v_mfma_f32_16x16x32_bf16 as the decode kernel does, with 16 query rows in
 // place of the GQA heads: the lane holding row l%16 keeps that row's softmax
-// state and 32 O^T accumulators per head.  A workgroup takes 16 rows of one
-// request and several query heads of one KV head; its four waves share
-// double-buffered LDS K/V tiles of 32 keys.  The layouts are described above
-// window_kernel.
+// state and 32 O^T accumulators per head.  A workgroup takes rows of one
+// request and query heads of one KV head, 128 (row, head) columns in all; its
+// four waves share double-buffered LDS K/V tiles.  The layouts are described
+// above window_kernel.
 
 #include <hip/hip_runtime.h>
 #include <hip/hip_fp16.h>
@@ -166,9 +166,8 @@ __global__ void __launch_bounds__(256) downdate_kernel(const uint16_t* __restric
 
 // ------------------------------------------------------ window attention ----
 
-constexpr int kRows = 16;    // query rows per wave
-constexpr int kBlk = 32;     // keys per block
 constexpr int kMaxB = 4096;  // requests handled by the in-workgroup planner
+constexpr int kTiles = 8;    // column tiles (16 query rows of one head) of a task
 
 struct WindowParams {
   const uint16_t* q;  // attention queries [total_q, Hq, 128]
@@ -180,6 +179,10 @@ struct WindowParams {
   // plain window attention
   uint16_t* out;
   float* out_lse;
+  // split form: partial states of the pieces, and the most pieces they hold
+  float* part_o;
+  float* part_ml;
+  int max_pieces;
   // fused rectification
   const uint16_t* src_q;
   const uint16_t* o_full;
@@ -199,159 +202,233 @@ struct WindowParams {
   float q_scale;  // sm_scale * log2(e)
 };
 
-// First row of request b that a kernel computes: 0 (plain form: every row),
-// or the first of the last min(len, M) rows, which the ring keeps (fused form).
-template <bool kRectify>
+enum WindowMode { kPlain = 0, kRectify = 1, kSplit = 2 };
+
+// First row of request b that a kernel computes: 0 (every row), or the first
+// of the last min(len, M) rows, which the ring keeps (fused form).
+template <int kMode>
 __device__ __forceinline__ int first_row(int len, int M) {
-  return kRectify ? (len > M ? len - M : 0) : 0;
+  return kMode == kRectify ? (len > M ? len - M : 0) : 0;
 }
 
 // Rows of request b the kernel computes; 0 for requests whose query or key
 // ranges fall outside the buffers the caller described, or with fewer keys
 // than queries.
-template <bool kRectify>
+template <int kMode>
 __device__ __forceinline__ int request_rows(const WindowParams& p, int b) {
   const int q0 = p.qo_indptr[b], q1 = p.qo_indptr[b + 1];
   const int k0 = p.kv_indptr[b], k1 = p.kv_indptr[b + 1];
   const int len = q1 - q0, kvlen = k1 - k0;
   const bool ok = q0 >= 0 && q1 <= p.total_q && k0 >= 0 && k1 <= p.kv_len_total && len > 0 && kvlen >= len;
-  return ok ? len - first_row<kRectify>(len, p.M) : 0;
+  return ok ? len - first_row<kMode>(len, p.M) : 0;
+}
+
+// Exclusive scan of one value per thread over a 256-thread workgroup; the
+// total goes to `total`.  s_tmp: kWaves entries; ends with a barrier.
+__device__ __forceinline__ int scan256(int v, int* s_tmp, int& total) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  int x = v;
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) {
+    const int y = __shfl_up(x, off);
+    if (lane >= off) x += y;
+  }
+  if (lane == 63) s_tmp[wave] = x;
+  __syncthreads();
+  int base = x - v;
+  total = 0;
+#pragma unroll
+  for (int w = 0; w < kWaves; ++w) {
+    if (w < wave) base += s_tmp[w];
+    total += s_tmp[w];
+  }
+  __syncthreads();
+  return base;
+}
+
+// The plan of a batch, derived by every workgroup: s_boff[b] = pieces of the
+// requests before b.  A piece is a block of kRowsT rows (plain and fused
+// forms) or one key chunk of such a block (split form: ceil(kvlen / chunk)
+// chunks per block).  Returns the chunk (split form).
+//
+// Split form: the number of key chunks must fit p.max_pieces partial states
+// and follows from the batch: with W = sum of blocks x keys and NB blocks,
+// chunk = W / (max_pieces - NB) rounded up to whole 64-key blocks gives at
+// most W / chunk + NB <= max_pieces pieces.  Requests whose query ranges
+// overlap can hold more row blocks than the caller's row count allows for:
+// with no room for them the chunk is kNoChunk, every piece is a whole block
+// and writes its result itself.
+constexpr int kNoChunk = 1 << 30;  // (a request has fewer keys)
+constexpr int kMinSplitKeys = 256;  // smallest chunk: a piece's prologue and state cost about as much
+
+template <int kMode, int kRowsT>
+__device__ __forceinline__ int plan_pieces(const WindowParams& p, int* s_boff, int* s_tmp) {
+  const int tid = threadIdx.x;
+  const int B = p.B;
+  const int per = ceil_div(B, 256);
+  const int b0 = min(B, tid * per), b1 = min(B, b0 + per);
+  int chunk = 0;
+  if (kMode == kSplit) {
+    int nb = 0;
+    long long w = 0;
+    for (int b = b0; b < b1; ++b) {
+      const int n = ceil_div(request_rows<kMode>(p, b), kRowsT);
+      nb += n;
+      w += static_cast<long long>(n) * (p.kv_indptr[b + 1] - p.kv_indptr[b]);
+    }
+    int total_nb;
+    scan256(nb, s_tmp, total_nb);
+    __shared__ long long s_w[kWaves];
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) w += __shfl_xor(w, off);
+    if ((tid & 63) == 0) s_w[tid >> 6] = w;
+    __syncthreads();
+    w = 0;
+#pragma unroll
+    for (int i = 0; i < kWaves; ++i) w += s_w[i];
+    const int room = p.max_pieces - total_nb;
+    const long long c = room > 0 ? ((w + room - 1) / room + 63) / 64 * 64 : kNoChunk;
+    chunk = static_cast<int>(min(max(c, static_cast<long long>(kMinSplitKeys)), static_cast<long long>(kNoChunk)));
+  }
+  int sum = 0;
+  for (int b = b0; b < b1; ++b) {
+    int n = ceil_div(request_rows<kMode>(p, b), kRowsT);
+    if (kMode == kSplit && n > 0) n *= ceil_div(p.kv_indptr[b + 1] - p.kv_indptr[b], chunk);
+    s_boff[b] = n;  // the count until the prefix replaces it below
+    sum += n;
+  }
+  int total;
+  int acc = scan256(sum, s_tmp, total);
+  for (int b = b0; b < b1; ++b) {
+    const int n = s_boff[b];
+    s_boff[b] = acc;
+    acc += n;
+  }
+  if (tid == 0) s_boff[B] = total;
+  __syncthreads();
+  return chunk;
+}
+
+// Largest b < B with s_boff[b] <= piece.
+__device__ __forceinline__ int request_of(const int* s_boff, int B, int piece) {
+  int lo = 0, hi = B - 1;
+  while (lo < hi) {
+    const int mid = (lo + hi + 1) >> 1;
+    if (s_boff[mid] <= piece) lo = mid;
+    else hi = mid - 1;
+  }
+  return lo;
 }
 
 // Sliding-window attention for GQA groups of any size: the windowed
-// FlashInfer pass (kRectify false) or the fused rectification of the rows
-// the ring keeps (kRectify true: a window of S keys, optionally the front
-// sink [0, min(F, E)) as a second key segment, P fed to the PV product as
-// bf16 hi + lo, and the downdate and ring write as epilogue).  A workgroup takes 16 consecutive query rows of one
-// request and 4 * HPW query heads of one KV head (HPW heads per wave), so
-// every 32-key K/V tile it stages in LDS serves 16 rows x 4 HPW heads.  Per
-// wave and block:
-//  * S^T = K Q^T: the A operand (K rows) is read once and used for the
-//    wave's HPW heads.  Tile t's MFMA row m = 4a + i holds key 8a + 4t + i,
-//    so the lane holding row (query) col ends up with the scores of keys
-//    8q .. 8q + 7 (q = lane / 16) -- consecutive keys, which is what the PV
-//    product's B operand needs.
-//  * O^T += V^T P^T: V stays token-major in LDS; the A operand of each
-//    16-dim tile, V^T[16 dt + col][8q .. 8q + 7], is two transposing LDS
-//    reads (ds_read_b64_tr_b16: in each 16-lane group, lane i receives
-//    element i & 3 of the 4-element vectors of lanes 4e + (i >> 2), e < 4),
-//    again shared by the wave's heads.
-// LDS layouts: K chunk c (16 bytes) of key k at position c ^ (4 ((k >> 3) &
-// 3) + (k & 3)) of its 256-byte row, which puts the 16 keys one A-operand
-// read touches on 16 different 16-byte bank groups; V row k at byte
-// 288 k + 128 (k >> 3) (rows padded to 288 bytes, each group of 8 keys a
-// further 128 bytes on): a transposing read takes 32 lanes per cycle, keys
-// 8a + 4h + (0..3) and 8a + 8 + 4h + (0..3) x 32 bytes, which this puts on
-// the 32 different 8-byte bank pairs of the 64 banks (with the padding alone
-// the two key groups collide), and its address stays an immediate offset
-// per 16-dim tile.
-// Key validity of a block is one 32-bit mask in LDS; a lane turns it into
-// the mask of its 8 keys with the row's window bounds by shifts.  The running
-// maximum is moved lazily (only when a block exceeds it by 2^8), which leaves
-// the result exact and skips most accumulator rescales.
+// FlashInfer pass (kPlain), the same over pieces of a row's keys with partial
+// results (kSplit, for batches with too few row blocks to fill the GPU), or
+// the fused rectification of the rows the ring keeps (kRectify: a window of S
+// keys, optionally the front sink [0, min(F, E)) as a second key segment, P
+// fed to the PV product as bf16 hi + lo, and the downdate and ring write as
+// epilogue).
+//
+// A task is 8 column tiles of one KV head: a tile is 16 consecutive query
+// rows of one query head, and the 8 are RT row tiles x 8 / RT heads, RT
+// picked from the GQA group so that no tile is wasted on an absent head (G >
+// 4: 16 rows x 8 heads; 3, 4: 32 x 4; 2: 64 x 2; 1: 128 x 1).  Each of the
+// four waves owns two of them, so every K and V operand a wave reads from LDS
+// feeds 32 columns whatever the group size.  K/V rows are staged in
+// double-buffered LDS tiles of kBlk keys: 64 (plain; one barrier and one
+// round of address work per 64 keys), or 32 (fused form, whose epilogue also
+// holds the full state's rows in LDS).  Per wave and 32 keys:
+//  * S^T = K Q^T: the A operand of score tile t, row m, is key 16 t + m; the
+//    lane holding column col ends up with the scores of keys 16 t + 4 quad +
+//    (0..3), quad = lane / 16.
+//  * O^T += V^T P^T: V stays token-major in LDS; the A operand of each 16-dim
+//    tile is two transposing LDS reads (ds_read_b64_tr_b16: in each 16-lane
+//    group, lane i receives element i & 3 of the 4-element vectors of lanes
+//    4e + (i >> 2), e < 4), the first of keys 4 quad + (0..3), the second of
+//    keys 16 + 4 quad + (0..3): the same order of keys as P has in the lane's
+//    B operand, so P goes from the score tiles to the PV product unmoved.
+// LDS layouts: K chunk c (16 bytes) of key k at position c ^ (k & 15) of its
+// 256-byte row; V row k at 288 k bytes.  A K read covers 16 consecutive keys
+// on 16 different chunk positions, also where the hardware pairs lanes of two
+// quads (rows padded to 272 bytes instead cost one conflict cycle per group
+// of 16 lanes there: 23% of the LDS cycles), and the 8 keys of a V read (two
+// quads) are 32 bytes apart in the banks.
+// What bounds it: per wave and 32 keys, 32 MFMAs (512 clocks) and about 105
+// other VALU instructions (670 clocks, the exponentials at a quarter of the
+// rate) that the SIMD's two waves overlap only partly: 1500 clocks per wave
+// and 32 keys, 800-850 TFLOP/s over long windows (a large bf16 matrix product
+// reaches 1200 on the same card).  Before every wave had two tiles, groups of
+// at most four heads read each operand for 16 columns only.  8 x 8192 rows,
+// 32 query heads, window 256 / 2048 (us), one tile per wave -> two: 4 heads
+// per group 655 / 3570 -> 577 / 2655; 1 head 1840 / 9470 -> 706 / 2930 (8
+// heads had two before: 549 / 2600).  The fused form, 8 x 512 kept rows,
+// 4 heads per group: 72 -> 62 us.
+// The running maximum is moved lazily (only when a block exceeds it by 2^8),
+// which leaves the result exact and skips most accumulator rescales.
 
-constexpr int kVRow = 18;  // 16-byte units per staged V row: 256 bytes + 32 of padding
-// 16-byte position of V row k in the staged tile
-__device__ __forceinline__ int v_row(int k) { return k * kVRow + 8 * (k >> 3); }
-constexpr int kVTile = kBlk * kVRow + 8 * (kBlk / 8 - 1);  // 16-byte units of a staged V tile
+constexpr int kKRow = 16;  // 16-byte units per staged K row
+constexpr int kVRow = 18;  // per staged V row: 256 + 32
 
-// Residency: the one-head-per-wave window pass fits 168 VGPRs, so it runs
-// three workgroups per CU (more waves per SIMD to overlap the softmax VALU
-// work with the MFMAs: 7% faster at GQA-4); the others need more registers.
-template <int HPW, bool kRectify>
-__global__ void __launch_bounds__(256, (HPW == 1 && !kRectify) ? 3 : 2) window_kernel(WindowParams p) {
-  // dynamic: s_boff[B + 1] row-block offsets, s_qo[B + 1] / s_kv[B + 1] the
+template <int RT, int kMode>
+__global__ void __launch_bounds__(256, 2) window_kernel(WindowParams p) {
+  constexpr bool kFused = kMode == kRectify;
+  constexpr int kHeads = kTiles / RT;   // query heads of a task
+  constexpr int kRowsT = 16 * RT;       // query rows of a task
+  constexpr int kBlk = kFused ? 32 : 64;  // keys per staged block
+  constexpr int kSub = kBlk / 32;
+  constexpr int kLd = kBlk / 16;  // keys each thread stages a chunk of
+  // dynamic: s_boff[B + 1] piece offsets, s_qo[B + 1] / s_kv[B + 1] the
   // request offsets (copies of qo_indptr / kv_indptr)
   extern __shared__ int s_dyn[];
   int* s_boff = s_dyn;
   int* s_qo = s_dyn + (p.B + 1);
   int* s_kv = s_dyn + 2 * (p.B + 1);
   __shared__ int s_part[kWaves];
-  __shared__ uint4 s_k[2][kBlk * 16];  // K rows of a 32-key block (swizzled)
-  __shared__ uint4 s_v[2][kVTile];  // V rows of the block (v_row layout)
-  __shared__ uint32_t s_okw[2][kWaves];  // per wave: bits of its 8 keys that have a pool row
+  __shared__ uint4 s_k[2][kBlk * kKRow];
+  __shared__ uint4 s_v[2][kBlk * kVRow];
+  __shared__ uint32_t s_bad[2][kWaves][2];  // per wave: its keys (of each 32) that have no pool row
 
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lane = tid & 63;
   const int quad = lane >> 4;
   const int col = lane & 15;
-
-  // ---- plan: s_boff[b] = sum over b' < b of ceil(rows(b') / 16) ----
   const int B = p.B;
-  const int per = ceil_div(B, 256);
-  {
-    int sum = 0;
-    for (int b = tid * per; b < min(B, (tid + 1) * per); ++b) {
-      const int n = ceil_div(request_rows<kRectify>(p, b), kRows);
-      s_boff[b] = n;  // the count until the prefix replaces it below
-      sum += n;
-    }
-    for (int b = tid; b <= B; b += 256) {
-      s_qo[b] = p.qo_indptr[b];
-      s_kv[b] = p.kv_indptr[b];
-    }
-    // exclusive scan of the per-thread sums: inclusive within each wave by
-    // lane shifts, then the four wave totals through LDS (one barrier)
-    int x = sum;
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-      const int y = __shfl_up(x, off);
-      if (lane >= off) x += y;
-    }
-    if (lane == 63) s_part[wave] = x;
-    __syncthreads();
-    int acc = x - sum, total = 0;
-#pragma unroll
-    for (int w = 0; w < kWaves; ++w) {
-      if (w < wave) acc += s_part[w];
-      total += s_part[w];
-    }
-    for (int b = tid * per; b < min(B, (tid + 1) * per); ++b) {
-      const int n = s_boff[b];
-      s_boff[b] = acc;
-      acc += n;
-    }
-    if (tid == 0) s_boff[B] = total;
-    __syncthreads();
+  for (int b = tid; b <= B; b += 256) {
+    s_qo[b] = p.qo_indptr[b];
+    s_kv[b] = p.kv_indptr[b];
   }
+  const int chunk = plan_pieces<kMode, kRowsT>(p, s_boff, s_part);
   const int Hq = p.Hq, Hkv = p.Hkv;
   const int G = Hq / Hkv;
-  constexpr int kHeadsPerTask = 4 * HPW;
-  // fused form: the full state's o rows of the task (row r, task head hh,
-  // 16-byte part c at r * kOfRow + 16 hh + c; rows padded by one part)
-  constexpr int kOfRow = kHeadsPerTask * 16 + 1;
-  __shared__ uint4 s_of[kRectify ? kRows * kOfRow : 1];
-  const int nchunks = ceil_div(G, kHeadsPerTask);
-  const int total_tasks = s_boff[B] * Hkv * nchunks;
+  // fused form: the full state's o rows of the task.  Pair e = row * kHeads +
+  // head takes 16 16-byte units from unit 16 e + (e >> 2) on (the extra unit
+  // per four pairs spreads the rows over the banks; a wave's direct copy
+  // fills four pairs, one contiguous 1 KiB run)
+  __shared__ uint4 s_of[kFused ? 128 * 16 + 32 : 1];
+  const int nchunks = ceil_div(G, kHeads);
+  const int per_piece = Hkv * nchunks;
+  const int total_tasks = s_boff[B] * per_piece;
   const uint32_t row_bytes = static_cast<uint32_t>(Hkv) * kHeadDim * 2;  // one pool row of K or V
   const unsigned pool_rows = static_cast<unsigned>(min(p.pool_tokens, static_cast<int64_t>(INT_MAX)));
   // keys [pos - wl, pos] form a row's window (wl < 0: [0, pos])
-  const int wl = kRectify ? p.S - 1 : p.window_left;
-  const bool sink = kRectify && p.sink_mode == 1 && p.F > 0;  // the front sink [0, min(F, E)) as well
-  // loader side: thread t stages 16-byte chunk t%16 of keys 2 (t/16) and 2 (t/16) + 1
-  const int ld_key = 2 * (tid >> 4), ld_chunk = tid & 15;
-  const int ld_pk0 = ld_key * 16 + (ld_chunk ^ (4 * ((ld_key >> 3) & 3) + (ld_key & 3)));
-  const int ld_pk1 = (ld_key + 1) * 16 + (ld_chunk ^ (4 * (((ld_key + 1) >> 3) & 3) + ((ld_key + 1) & 3)));
-  const int ld_pv0 = v_row(ld_key) + ld_chunk;
-  const int ld_pv1 = v_row(ld_key + 1) + ld_chunk;
-  // compute side: K A-operand positions (tile t, k-step s) and V^T read
-  // addresses (16-dim tile dt, half h) of this lane
-  int pk[2][4];
+  const int wl = kFused ? p.S - 1 : p.window_left;
+  const bool sink = kFused && p.sink_mode == 1 && p.F > 0;  // the front sink [0, min(F, E)) as well
+  // loader side: thread t stages 16-byte chunk t%16 of keys t/16 + 16 i
+  const int ld_key = tid >> 4, ld_chunk = tid & 15;
+  u32x4_t* const ld_k = reinterpret_cast<u32x4_t*>(&s_k[0][0]) + ld_key * kKRow + (ld_chunk ^ ld_key);
+  u32x4_t* const ld_v = reinterpret_cast<u32x4_t*>(&s_v[0][0]) + ld_key * kVRow + ld_chunk;
+  // compute side: this lane's K row (key col) and V^T read position (key 4
+  // quad + (col >> 2), dims 4 (col & 3) ..)
+  const uint4* rd_k[4];  // by k-step
 #pragma unroll
-  for (int t = 0; t < 2; ++t) {
-    const int key = 8 * (col >> 2) + 4 * t + (col & 3);
-    const int sw = 4 * ((key >> 3) & 3) + (key & 3);
-#pragma unroll
-    for (int s = 0; s < 4; ++s) pk[t][s] = key * 16 + ((4 * s + quad) ^ sw);
-  }
-  // V^T: lane j = col of group quad reads key 8 quad + 4 h + (j >> 2), dims
-  // 16 dt + 4 (j & 3) .. + 3: element offset pv[h] + 16 dt of the V tile
-  int pv[2];
-#pragma unroll
-  for (int h = 0; h < 2; ++h) pv[h] = v_row(8 * quad + 4 * h + (col >> 2)) * 8 + 4 * (col & 3);
+  for (int s = 0; s < 4; ++s) rd_k[s] = &s_k[0][0] + col * kKRow + ((4 * s + quad) ^ col);
+  const uint16_t* const rd_v =
+      reinterpret_cast<const uint16_t*>(&s_v[0][0]) + (4 * quad + (col >> 2)) * (kVRow * 8) + 4 * (col & 3);
+  // the wave's tiles c = 0, 1: task head and first row in the task
+  const int th0 = (2 * wave) / RT, th1 = (2 * wave + 1) / RT;
+  const int tr0 = 16 * ((2 * wave) % RT), tr1 = 16 * ((2 * wave + 1) % RT);
 
-  // Task order, by form (measured at config 4's prefill shape):
+  // Task order, by form (measured at 64 requests x 8192 rows, S = 256):
   //  * windowed (plain, window_left >= 0): (KV head, head chunk) major, row
   //    block minor, and within each full round of the grid XCD x (the
   //    workgroups w with w % 8 == x, as the dispatcher deals them) takes the
@@ -360,392 +437,426 @@ __global__ void __launch_bounds__(256, (HPW == 1 && !kRectify) ? 3 : 2) window_k
   //    put them on different XCDs and fetched each K/V row about four times);
   //  * fused: row-block order (the KV heads of a row block together), XCD
   //    eighths as above (2-3% faster than round-robin; head-major was slower);
-  //  * causal (window_left < 0): row-block order dealt round-robin.  Its
-  //    tasks grow with the row block, and a workgroup keeps its offset within
-  //    every round, so a head-major order would give some workgroups only the
-  //    longest tasks.
+  //  * causal (window_left < 0) and split: row-block order dealt
+  //    round-robin.  Causal tasks grow with the row block, and a workgroup
+  //    keeps its offset within every round, so a head-major order would give
+  //    some workgroups only the longest tasks.
   const int grid = gridDim.x;
   const int eighth = grid / 8;
-  const int nblocks = s_boff[B];
-  const bool head_major = !kRectify && wl >= 0;
-  const bool by_xcd = (kRectify || wl >= 0) && grid % 8 == 0;
+  const int npieces = s_boff[B];
+  const bool head_major = kMode == kPlain && wl >= 0;
+  const bool by_xcd = (kFused || (kMode == kPlain && wl >= 0)) && grid % 8 == 0;
   for (int task = blockIdx.x; task < total_tasks; task += grid) {
     __syncthreads();  // the previous task's waves are done with the tiles
     const int round0 = task - static_cast<int>(blockIdx.x);
     const int t = (by_xcd && round0 + grid <= total_tasks)
                       ? round0 + (static_cast<int>(blockIdx.x) % 8) * eighth + static_cast<int>(blockIdx.x) / 8
                       : task;
-    int blk, hc;  // row block; KV head * nchunks + head chunk
+    int piece, hc;  // piece; KV head * nchunks + head chunk
     if (head_major) {
-      hc = t / nblocks;
-      blk = t - hc * nblocks;
+      hc = t / npieces;
+      piece = t - hc * npieces;
     } else {
-      blk = t / (Hkv * nchunks);
-      hc = t - blk * Hkv * nchunks;
+      piece = t / per_piece;
+      hc = t - piece * per_piece;
     }
     const int hkv = hc / nchunks;
-    const int hg0 = kHeadsPerTask * (hc - hkv * nchunks) + HPW * wave;  // first head of this wave in the group
-    int lo = 0, hi = B - 1;  // request of this row block: largest b with s_boff[b] <= blk
-    while (lo < hi) {
-      const int mid = (lo + hi + 1) >> 1;
-      if (s_boff[mid] <= blk) lo = mid;
-      else hi = mid - 1;
-    }
-    const int b = lo;
+    const int hg0 = kHeads * (hc - hkv * nchunks);  // first head of the task in the group
+    const int b = request_of(s_boff, B, piece);
     const int len = s_qo[b + 1] - s_qo[b];
     const int kvlen = s_kv[b + 1] - s_kv[b];
     const int64_t kv_begin = s_kv[b];
-    const int r_local = first_row<kRectify>(len, p.M) + kRows * (blk - s_boff[b]);
-    const int nrows = min(kRows, len - r_local);
+    int blk = piece - s_boff[b], key_lo = 0, key_hi = INT_MAX;  // row block and key chunk
+    if (kMode == kSplit) {  // chunk-major: the row blocks that share a chunk's keys together
+      const int nb = ceil_div(len, kRowsT);
+      const int ch = blk / nb;
+      blk -= ch * nb;
+      key_lo = ch * chunk;
+      key_hi = key_lo + min(chunk, kvlen - key_lo);
+    }
+    const int r_local = first_row<kMode>(len, p.M) + kRowsT * blk;
+    const int nrows = min(kRowsT, len - r_local);
     const int pos0 = kvlen - len + r_local;
     const int pos_last = pos0 + nrows - 1;
-    const bool row_ok = col < nrows;
-    const int pos = pos0 + col;  // this lane's row position
-    const int64_t grow = static_cast<int64_t>(s_qo[b]) + r_local + (row_ok ? col : 0);
-    const int w_lo = wl < 0 ? 0 : max(pos - wl, 0);  // this row's window [w_lo, pos]
+    if (kMode == kSplit && key_lo > pos_last) continue;  // (past every row: the combine skips it too)
+    // tile c of the wave: lane's row in the task, position, first key of its window
+    const bool live0 = hg0 + th0 < G && tr0 < nrows, live1 = hg0 + th1 < G && tr1 < nrows;
+    const bool live = live0 || live1;
+    int row[2], wlo[2];
+    bool row_ok[2];
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+      row[c] = (c == 0 ? tr0 : tr1) + col;
+      row_ok[c] = row[c] < nrows && (c == 0 ? live0 : live1);
+      wlo[c] = wl < 0 ? 0 : max(pos0 + row[c] - wl, 0);
+    }
+    // first and last row of the wave's tiles (uniform), for the mask-free test
+    const int rf = min(tr0, tr1), rl = min(max(tr0, tr1) + 15, nrows - 1);
+    const int wlo_f = wl < 0 ? 0 : max(pos0 + rf - wl, 0), wlo_l = wl < 0 ? 0 : max(pos0 + rl - wl, 0);
     // this request's kv_indices; entry offsets fit 32 bits (fewer than 2^30
     // entries, checked on the host), so a load is a uniform base plus a
     // 32-bit lane offset
     const char* kvi = reinterpret_cast<const char*>(p.kv_indices + kv_begin);
+    const uint32_t last4 = 4u * static_cast<uint32_t>(kvlen - 1);
     auto index_at = [&](int key) -> int {  // entry of a key, clamped into the request
-      return *reinterpret_cast<const int*>(kvi + min(static_cast<uint32_t>(key), static_cast<uint32_t>(kvlen - 1)) * 4u);
+      return *reinterpret_cast<const int*>(kvi + min(static_cast<uint32_t>(key) * 4u, last4));
     };
     // The entries of the first segment's first two blocks (the loader's keys)
     // go out first, ahead of the Q rows and the epilogue's inputs: the first
     // K/V loads then wait for these entries only, not for everything issued
     // before them (the memory counter retires loads in order).
     const int seg_first = sink ? 0 : 1;
-    const int lo_first = seg_first == 0 ? 0 : (wl < 0 ? 0 : max(pos0 - wl, 0));
-    int pre_raw[4];
+    const int lo_first = seg_first == 0 ? 0 : max(wl < 0 ? 0 : max(pos0 - wl, 0), key_lo);
+    int pre_raw[2][kLd];
 #pragma unroll
-    for (int t = 0; t < 4; ++t) pre_raw[t] = index_at(lo_first + (t >> 1) * kBlk + ld_key + (t & 1));
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+      for (int i = 0; i < kLd; ++i) pre_raw[u][i] = index_at(lo_first + u * kBlk + ld_key + 16 * i);
     __builtin_amdgcn_sched_barrier(0);  // (kept ahead of the loads below)
     // fused form: the epilogue's inputs that do not depend on the attention,
     // loaded now so that their latency hides behind it
+    auto grow = [&](int r) { return static_cast<int64_t>(s_qo[b]) + r_local + (r < nrows ? r : 0); };
+    const int64_t grow0 = grow(row[0]), grow1 = grow(row[1]);
     int req = 0, before = 0;
-    float lse_full[HPW];
-    if (kRectify) {
+    float lse_full[2] = {0.0f, 0.0f};
+    if (kFused) {
       req = p.req_ids[b];
       const bool req_ok = req >= 0 && req < p.R;
       before = p.rl_by_batch ? p.request_length[b] : p.request_length[req_ok ? req : 0];
-#pragma unroll
-      for (int i = 0; i < HPW; ++i) lse_full[i] = p.lse_full[grow * Hq + hkv * G + min(hg0 + i, G - 1)];
+      lse_full[0] = p.lse_full[grow0 * Hq + hkv * G + min(hg0 + th0, G - 1)];
+      lse_full[1] = p.lse_full[grow1 * Hq + hkv * G + min(hg0 + th1, G - 1)];
     }
-    const int nheads = __builtin_amdgcn_readfirstlane(max(0, min(HPW, G - hg0)));  // heads this wave computes
     // Fused form: the task's pre-RoPE query rows (copied into the ring with
     // the q_post NaN marker) and the full state's o rows (into s_of for the
-    // epilogue) -- 16 rows x kHeadsPerTask heads x 16 parts of 16 bytes,
-    // kHeadsPerTask rounds of one part per thread -- move with the K/V
-    // stream, so that this traffic overlaps the compute-bound key blocks
-    // instead of adding an HBM-bound load round after them (every workgroup
-    // runs its task in step with the others).  A round's loads go out behind
-    // a block's K/V loads; its query part is stored when the next block is
-    // staged, and its o part is copied straight into LDS
-    // (global_load_lds_dwordx4: no registers; waited for at the next
-    // block's staging and barrier).  Round k, thread t: row (16 k + t / 16) /
-    // kHeadsPerTask, task head (t / 16) % kHeadsPerTask, part t % 16 -- the
-    // 64 lanes of a wave take 4 heads x 16 parts of one row, a contiguous
-    // 1 KiB run of s_of, which is the run a wave's copy fills.
-    const int cq_hh = (tid >> 4) % kHeadsPerTask;
+    // epilogue) -- 128 (row, head) pairs x 16 parts of 16 bytes, 8 rounds of
+    // one part per thread -- move with the K/V stream, so that this traffic
+    // overlaps the compute-bound key blocks instead of adding an HBM-bound
+    // load round after them (every workgroup runs its task in step with the
+    // others).  A round's loads go out behind a block's K/V loads; its query
+    // part is stored when the next block is staged, and its o part is copied
+    // straight into LDS (global_load_lds_dwordx4: no registers; waited for at
+    // the next block's staging and barrier).  Round k, thread t: pair 16 k +
+    // t / 16, part t % 16.
+    constexpr int kCq = 8;
     const int cq_part = tid & 15;
-    const int cq_h = kHeadsPerTask * (hc - hkv * nchunks) + cq_hh;  // its head in the group
-    const bool cq_req = kRectify && req >= 0 && req < p.R;
+    const bool cq_req = kFused && req >= 0 && req < p.R;
     int cq = 0;               // rounds issued (uniform)
     bool cq_pending = false;  // round cq - 1 loaded, its query part not yet stored
     uint4 cq_src = make_uint4(0, 0, 0, 0);
-    auto cq_row = [&](int k) { return (16 * k + (tid >> 4)) / kHeadsPerTask; };
     auto cq_issue = [&](int k) {
-      const int r = min(cq_row(k), nrows - 1);  // (rows past the block: a valid address, not stored)
-      const int64_t e = ((static_cast<int64_t>(s_qo[b]) + r_local + r) * Hq + hkv * G + min(cq_h, G - 1)) * kHeadDim +
-                        8 * cq_part;
-      cq_src = *reinterpret_cast<const uint4*>(p.src_q + e);
-      // the wave's run: row (16 k + 4 wave) / kHeadsPerTask, heads from (4 wave) % kHeadsPerTask
-      uint4* run = &s_of[((16 * k + 4 * wave) / kHeadsPerTask) * kOfRow + 16 * ((4 * wave) % kHeadsPerTask)];
-      __builtin_amdgcn_global_load_lds(static_cast<const void*>(p.o_full + e),
+      const int e = 16 * k + (tid >> 4);
+      const int r = min(e / kHeads, nrows - 1);  // (rows past the block: a valid address, not stored)
+      const int64_t at = ((static_cast<int64_t>(s_qo[b]) + r_local + r) * Hq + hkv * G + min(hg0 + e % kHeads, G - 1)) *
+                             kHeadDim + 8 * cq_part;
+      cq_src = *reinterpret_cast<const uint4*>(p.src_q + at);
+      uint4* run = &s_of[(16 * k + 4 * wave) * 16 + (16 * k + 4 * wave) / 4];  // the wave's four pairs
+      __builtin_amdgcn_global_load_lds(static_cast<const void*>(p.o_full + at),
                                        (__attribute__((address_space(3))) void*)(run), 16, 0, 0);
     };
     auto cq_store = [&](int k) {
-      const int r = cq_row(k);
-      if (cq_req && r < nrows && cq_h < G) {
+      const int e = 16 * k + (tid >> 4);
+      const int r = e / kHeads, h = hg0 + e % kHeads;
+      if (cq_req && r < nrows && h < G) {
         const int slot = static_cast<int>((static_cast<int64_t>(max(before, 0)) + r_local + r) % p.M);
-        const int64_t e = ((static_cast<int64_t>(req) * p.M + slot) * Hq + hkv * G + cq_h) * kHeadDim + 8 * cq_part;
-        *reinterpret_cast<uint4*>(p.q_cache + e) = cq_src;
+        const int64_t at = ((static_cast<int64_t>(req) * p.M + slot) * Hq + hkv * G + h) * kHeadDim + 8 * cq_part;
+        *reinterpret_cast<uint4*>(p.q_cache + at) = cq_src;
         if (p.q_post_cache != nullptr)
-          *reinterpret_cast<uint4*>(p.q_post_cache + e) = make_uint4(0x7fc07fc0u, 0x7fc07fc0u, 0x7fc07fc0u, 0x7fc07fc0u);
+          *reinterpret_cast<uint4*>(p.q_post_cache + at) = make_uint4(0x7fc07fc0u, 0x7fc07fc0u, 0x7fc07fc0u, 0x7fc07fc0u);
       }
     };
 
-    // Q rows of the wave's heads (B operands): lane (quad, col) holds
-    // Q[row col][8 (4s + quad) .. +8].  A lane past the block's rows reads
-    // the block's first row and an absent head reads the group's first head
-    // (valid data, never zeroed): every score of such a lane is masked
-    // (kmask 0), an absent head is never stored, and each head keeps its own
-    // softmax state.  With no select on the loaded values no wait follows
-    // the loads: the Q rows and the first entries are one round of loads.
-    uint4 qreg[HPW][4];
+    // Q rows of the wave's tiles (B operands): lane (quad, col) holds
+    // Q[row][8 (4s + quad) .. +8].  A lane past the task's rows reads its
+    // first row and an absent head the group's last head (valid data, never
+    // zeroed): such a lane's results are never stored, and each column keeps
+    // its own softmax state.  With no select on the loaded values no wait
+    // follows the loads: the Q rows and the first entries are one round.
+    uint4 qreg[2][4];
 #pragma unroll
-    for (int i = 0; i < HPW; ++i) {
-      const int h = hkv * G + (hg0 + i < G ? hg0 + i : 0);
-      const uint16_t* qp = p.q + (grow * Hq + h) * kHeadDim;
+    for (int c = 0; c < 2; ++c) {
+      const int h = hkv * G + min(hg0 + (c == 0 ? th0 : th1), G - 1);
+      const uint16_t* qp = p.q + ((c == 0 ? grow0 : grow1) * Hq + h) * kHeadDim;
 #pragma unroll
-      for (int s = 0; s < 4; ++s) qreg[i][s] = *reinterpret_cast<const uint4*>(qp + 8 * (4 * s + quad));
+      for (int s = 0; s < 4; ++s) qreg[c][s] = *reinterpret_cast<const uint4*>(qp + 8 * (4 * s + quad));
     }
 
-    // l[h]: the softmax row sums.  Plain form: the lane's fp32 partial sums
-    // in l[h][0] (reduced over the row's four lanes at the end).  Fused form:
-    // accumulated by MFMAs with an all-ones A operand over P = hi + lo (every
-    // element of the lane's l[h] then holds its row's sum), off the VALU; the
-    // plain form cannot do that, since its P is bf16 hi alone and the sum of
-    // that is ~2^-9 off per key, beyond what its lse output allows.
-    float m[HPW];
-    f32x4_t acc[HPW][8], l[HPW];
+    // l[c]: the softmax row sums.  Plain form: the lane's fp32 partial sums
+    // in l[c][0] (reduced over the column's four lanes at the end).  Fused
+    // form: accumulated by MFMAs with an all-ones A operand over P = hi + lo
+    // (every element of the lane's l[c] then holds its column's sum), off the
+    // VALU; the plain form cannot do that, since its P is bf16 hi alone and
+    // the sum of that is ~2^-9 off per key, beyond what its lse output allows.
+    // vt[c]: the scaled score past which m[c] moves (-inf: none seen yet).
+    float m[2] = {kNegBig, kNegBig}, vt[2] = {-INFINITY, -INFINITY};
+    f32x4_t acc[2][8], l[2];
 #pragma unroll
-    for (int i = 0; i < HPW; ++i) {
-      m[i] = kNegBig;
-      l[i] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int c = 0; c < 2; ++c) {
+      l[c] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-      for (int dt = 0; dt < 8; ++dt) acc[i][dt] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+      for (int dt = 0; dt < 8; ++dt) acc[c][dt] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
     }
 
     const char* kbase = reinterpret_cast<const char*>(p.k + static_cast<int64_t>(hkv) * kHeadDim + ld_chunk * 8);
-    const char* vbase = reinterpret_cast<const char*>(p.v + static_cast<int64_t>(hkv) * kHeadDim + ld_chunk * 8);
-    bool fresh = true;  // no block computed yet: the first sets m without a rescale
-    auto ld = [&](const char* base, int r) -> uint4 {  // one v_mad_u64_u32 per address
-      return *reinterpret_cast<const uint4*>(base + static_cast<uint64_t>(static_cast<uint32_t>(max(r, 0))) * row_bytes);
+    const int64_t v_minus_k = reinterpret_cast<const char*>(p.v) - reinterpret_cast<const char*>(p.k);
+    // the loader's K/V chunks of the block in flight (ok: bit i set if key i
+    // has a row) and the raw indices of the block after it
+    uint32_t ok = 0;
+    int rn[kLd];
+    u32x4_t kq[kLd], vq[kLd];
+    auto load_block = [&](int base, int end, const int (&raw)[kLd]) {
+      ok = 0;
+#pragma unroll
+      for (int i = 0; i < kLd; ++i) {
+        const bool in = base + ld_key + 16 * i < end && static_cast<unsigned>(raw[i]) < pool_rows;
+        ok |= in ? 1u << i : 0u;
+        const char* at = kbase + static_cast<uint64_t>(static_cast<uint32_t>(in ? raw[i] : 0)) * row_bytes;
+        kq[i] = *reinterpret_cast<const u32x4_t*>(at);
+        vq[i] = *reinterpret_cast<const u32x4_t*>(at + v_minus_k);
+      }
     };
-    // the loader's K/V chunks of the block in flight (rc0/rc1: their rows,
-    // -1: masked) and the raw indices of the block after it
-    int rc0 = -1, rc1 = -1, rn0 = 0, rn1 = 0;
-    uint4 kq0 = make_uint4(0, 0, 0, 0), kq1 = kq0, vq0 = kq0, vq1 = kq0;
     {
       // the first segment's block 0 goes in flight here, right behind the Q
       // rows (issued in the segment loop, its loads would wait for every
       // load before them: the loop's entry joins the counts)
-      const int hi_first = seg_first == 0 ? min(p.F, max(pos_last - wl, 0)) : pos_last + 1;
+      const int hi_first = min(seg_first == 0 ? min(p.F, max(pos_last - wl, 0)) : pos_last + 1, key_hi);
       if (hi_first > lo_first) {
-        const int k0 = lo_first + ld_key;
-        rc0 = (k0 < hi_first && static_cast<unsigned>(pre_raw[0]) < pool_rows) ? pre_raw[0] : -1;
-        rc1 = (k0 + 1 < hi_first && static_cast<unsigned>(pre_raw[1]) < pool_rows) ? pre_raw[1] : -1;
-        kq0 = ld(kbase, rc0);
-        kq1 = ld(kbase, rc1);
-        vq0 = ld(vbase, rc0);
-        vq1 = ld(vbase, rc1);
-        rn0 = pre_raw[2];
-        rn1 = pre_raw[3];
+        load_block(lo_first, hi_first, pre_raw[0]);
+#pragma unroll
+        for (int i = 0; i < kLd; ++i) rn[i] = pre_raw[1][i];
       }
     }
     // segment 0: the front sink [0, min(F, w_lo)) of each row (fused form,
     // sink_mode 1); segment 1: the window [w_lo, pos]
     for (int seg = seg_first; seg < 2; ++seg) {
-      const int seg_lo = seg == 0 ? 0 : (wl < 0 ? 0 : max(pos0 - wl, 0));
-      const int seg_hi = seg == 0 ? min(p.F, max(pos_last - wl, 0)) : pos_last + 1;
-      const int r_lo = seg == 0 ? 0 : w_lo;  // this row's keys in the segment: [r_lo, r_hi)
-      const int r_hi = seg == 0 ? min(p.F, w_lo) : pos + 1;
+      const int seg_lo = seg == 0 ? 0 : max(wl < 0 ? 0 : max(pos0 - wl, 0), key_lo);
+      const int seg_hi = min(seg == 0 ? min(p.F, max(pos_last - wl, 0)) : pos_last + 1, key_hi);
       const int nblk = seg_hi > seg_lo ? ceil_div(seg_hi - seg_lo, kBlk) : 0;
-      // The loader's key ld_key + t of block i: its kv_indices entry (the load
-      // only, index clamped into the request) and, checked later, its pool row
-      // (-1: masked).  An index is loaded one block before it is checked, so
-      // the wait for it never includes K/V loads issued after it (the memory
-      // counter retires in order).
-      auto index_of = [&](int i, int t) -> int { return index_at(seg_lo + i * kBlk + ld_key + t); };
-      auto row_of = [&](int i, int t, int raw) -> int {
-        const int key = seg_lo + i * kBlk + ld_key + t;
-        return (key < seg_hi && static_cast<unsigned>(raw) < pool_rows) ? raw : -1;
-      };
+      // keys every row of the wave attends to, and keys any of them does
+      const int all_lo = seg == 0 ? 0 : wlo_l, all_hi = seg == 0 ? min(p.F, wlo_f) : pos0 + rf + 1;
+      const int any_lo = seg == 0 ? 0 : wlo_f, any_hi = seg == 0 ? min(p.F, wlo_l) : pos0 + rl + 1;
       if (seg != seg_first && nblk > 0) {  // (the first segment's block 0 is in flight)
-        rc0 = row_of(0, 0, index_of(0, 0));
-        rc1 = row_of(0, 1, index_of(0, 1));
-        kq0 = ld(kbase, rc0);
-        kq1 = ld(kbase, rc1);
-        vq0 = ld(vbase, rc0);
-        vq1 = ld(vbase, rc1);
-        rn0 = index_of(1, 0);
-        rn1 = index_of(1, 1);
+        int raw[kLd];
+#pragma unroll
+        for (int i = 0; i < kLd; ++i) raw[i] = index_at(seg_lo + ld_key + 16 * i);
+        load_block(seg_lo, seg_hi, raw);
+#pragma unroll
+        for (int i = 0; i < kLd; ++i) rn[i] = index_at(seg_lo + kBlk + ld_key + 16 * i);
       }
-      for (int i = 0; i < nblk; ++i) {
-        const int buf = i & 1;
-        // stage block i: K and V rows (V of masked keys zeroed), key validity bits
+      for (int blk_i = 0; blk_i < nblk; ++blk_i) {
+        const int buf = blk_i & 1;
+        const int base = seg_lo + blk_i * kBlk;
+        // stage the block: K and V rows (V of masked keys zeroed: P is 0 there, V may be NaN)
         {
-          s_k[buf][ld_pk0] = kq0;
-          s_k[buf][ld_pk1] = kq1;
-          const uint64_t b0 = __ballot(rc0 >= 0), b1 = __ballot(rc1 >= 0);
-          if ((b0 & b1) != ~0ull) {  // a masked key in the wave's rows: zero its V row (P is 0 there, V may be NaN)
-            const uint32_t z0 = rc0 >= 0 ? 0xffffffffu : 0u, z1 = rc1 >= 0 ? 0xffffffffu : 0u;
-            vq0 = make_uint4(vq0.x & z0, vq0.y & z0, vq0.z & z0, vq0.w & z0);
-            vq1 = make_uint4(vq1.x & z1, vq1.y & z1, vq1.z & z1, vq1.w & z1);
+          const bool all_ok = __all(ok == (1u << kLd) - 1u);
+          if (!all_ok) {
+#pragma unroll
+            for (int i = 0; i < kLd; ++i) {
+              const uint32_t z = (ok >> i) & 1 ? 0xffffffffu : 0u;
+              vq[i] &= u32x4_t{z, z, z, z};
+            }
           }
-          s_v[buf][ld_pv0] = vq0;
-          s_v[buf][ld_pv1] = vq1;
-          if (kRectify && cq_pending) {
+#pragma unroll
+          for (int i = 0; i < kLd; ++i) {
+            ld_k[buf * (kBlk * kKRow) + 16 * i * kKRow] = kq[i];
+            ld_v[buf * (kBlk * kVRow) + 16 * i * kVRow] = vq[i];
+          }
+          if (kFused && cq_pending) {
             cq_store(cq - 1);
             cq_pending = false;
           }
-          if (lane == 0) {
-            // lanes 16 r hold keys 8 wave + 2 r and 8 wave + 2 r + 1
-            uint32_t bits = 0;
+          uint32_t bad[2] = {0, 0};  // lanes 16 r: key 16 i + 4 wave + r, bit 16 (i & 1) + 4 wave + r of word i / 2
+          if (!all_ok) {
 #pragma unroll
-            for (int r = 0; r < 4; ++r)
-              bits |= static_cast<uint32_t>(((b0 >> (16 * r)) & 1) | (((b1 >> (16 * r)) & 1) << 1)) << (2 * r);
-            s_okw[buf][wave] = bits;
+            for (int i = 0; i < kLd; ++i) {
+              const uint64_t no = __ballot(((ok >> i) & 1) == 0);
+#pragma unroll
+              for (int r = 0; r < 4; ++r)
+                bad[i >> 1] |= static_cast<uint32_t>((no >> (16 * r)) & 1) << (16 * (i & 1) + 4 * wave + r);
+            }
+          }
+          if (lane == 0) {
+            s_bad[buf][wave][0] = bad[0];
+            s_bad[buf][wave][1] = bad[1];
           }
         }
-        __syncthreads();  // block i visible; every wave is done with block i - 2 (same buffer)
-        // block i + 1 in flight while block i is computed
-        if (i + 1 < nblk) {
-          rc0 = row_of(i + 1, 0, rn0);
-          rc1 = row_of(i + 1, 1, rn1);
-          kq0 = ld(kbase, rc0);
-          kq1 = ld(kbase, rc1);
-          vq0 = ld(vbase, rc0);
-          vq1 = ld(vbase, rc1);
-          rn0 = index_of(i + 2, 0);  // clamped: harmless past the last block
-          rn1 = index_of(i + 2, 1);
+        __syncthreads();  // the block is visible; every wave is done with the block before last (same buffer)
+        // the next block in flight while this one is computed
+        if (blk_i + 1 < nblk) {
+          load_block(base + kBlk, seg_hi, rn);
+#pragma unroll
+          for (int i = 0; i < kLd; ++i) rn[i] = index_at(base + 2 * kBlk + ld_key + 16 * i);  // (clamped)
         }
-        if (kRectify && cq < kHeadsPerTask) {
+        if (kFused && cq < kCq) {
           cq_issue(cq);
           ++cq;
           cq_pending = true;
         }
-        if (nheads == 0) continue;
-        const int base = seg_lo + i * kBlk;
-
-        // K A operands of both score tiles (row m = 4a + i <-> key 8a + 4t + i)
-        // and V A operands of the eight 16-dim tiles, all issued up front
-        uint4 ka[2][4];
+        if (!live) continue;
+        // sub-blocks of 32 keys that any of the wave's rows attends to
+        const int s_lo = (any_lo - base) >> 5, s_hi = min(seg_hi, any_hi) - base;  // (s_lo: arithmetic shift)
 #pragma unroll
-        for (int t = 0; t < 2; ++t)
+        for (int sub = 0; sub < kSub; ++sub) {
+          if (sub < s_lo || 32 * sub >= s_hi) continue;
+          const int kb = base + 32 * sub;
+          const int kt = buf * (kBlk * kKRow) + sub * (32 * kKRow);
+          const uint16_t* vtile = rd_v + (buf * (kBlk * kVRow) + sub * (32 * kVRow)) * 8;
+          uint32_t bad = 0;
 #pragma unroll
-          for (int s = 0; s < 4; ++s) ka[t][s] = s_k[buf][pk[t][s]];
-        const uint16_t* vtile = reinterpret_cast<const uint16_t*>(&s_v[buf][0]);
-        bf16x8_t va[8];
-#pragma unroll
-        for (int dt = 0; dt < 8; ++dt)
-          va[dt] = __builtin_shufflevector(lds_read_tr16(vtile + pv[0] + 16 * dt), lds_read_tr16(vtile + pv[1] + 16 * dt),
-                                           0, 1, 2, 3, 4, 5, 6, 7);
-        // mask of the lane's keys 8 quad + e: a pool row, and inside [r_lo, r_hi)
-        uint32_t kmask = s_okw[buf][quad];
-        {
-          const int k0 = base + 8 * quad;
-          const int lo_e = min(max(r_lo - k0, 0), 8), hi_e = min(max(r_hi - k0, 0), 8);
-          kmask &= ((1u << hi_e) - 1u) & ~((1u << lo_e) - 1u);
-          if (!row_ok) kmask = 0;
-        }
-        // blocks inside every row's range with every key present need no masks
-        const bool full = !__any(kmask != 0xffu);
-        // raw scores of both tiles and every head, the four accumulation chains
-        // interleaved (an absent head is computed but never stored)
-        f32x4_t c4[HPW][2];
-#pragma unroll
-        for (int h = 0; h < HPW; ++h)
-#pragma unroll
-          for (int t = 0; t < 2; ++t) c4[h][t] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-        for (int s = 0; s < 4; ++s)
+          for (int w = 0; w < kWaves; ++w) bad |= s_bad[buf][w][sub];
+          bad = __builtin_amdgcn_readfirstlane(bad);
+          uint4 ka[2][4];
 #pragma unroll
           for (int t = 0; t < 2; ++t)
 #pragma unroll
-            for (int h = 0; h < HPW; ++h)
-              c4[h][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(ka[t][s]), as_bf16x8(qreg[h][s]), c4[h][t],
-                                                                0, 0, 0);
-        if (!full) {  // masked keys -> -inf, the lane's eight bits decoded once for all heads
+            for (int s = 0; s < 4; ++s) ka[t][s] = rd_k[s][kt + 16 * t * kKRow];
+          bf16x8_t va[8];
 #pragma unroll
-          for (int e = 0; e < 8; ++e) {
-            const bool keep = (kmask >> e) & 1;
+          for (int dt = 0; dt < 8; ++dt)
+            va[dt] = __builtin_shufflevector(lds_read_tr16(vtile + 16 * dt), lds_read_tr16(vtile + 16 * kVRow * 8 + 16 * dt),
+                                             0, 1, 2, 3, 4, 5, 6, 7);
+          // raw scores, the four accumulation chains interleaved (a tile
+          // without rows is computed but never stored)
+          f32x4_t c4[2][2];
 #pragma unroll
-            for (int h = 0; h < HPW; ++h) c4[h][e >> 2][e & 3] = keep ? c4[h][e >> 2][e & 3] : -INFINITY;
+          for (int c = 0; c < 2; ++c)
+#pragma unroll
+            for (int t = 0; t < 2; ++t) c4[c][t] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+          for (int s = 0; s < 4; ++s)
+#pragma unroll
+            for (int t = 0; t < 2; ++t) {
+#pragma unroll
+              for (int c = 0; c < 2; ++c)
+                c4[c][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(ka[t][s]), as_bf16x8(qreg[c][s]), c4[c][t], 0, 0, 0);
+            }
+          // keys inside every row's range, all present, need no masks
+          if (kb < all_lo || kb + 32 > all_hi || bad != 0) {
+#pragma unroll
+            for (int c = 0; c < 2; ++c) {
+              const int pos = pos0 + row[c];
+              const int r_lo = seg == 0 ? 0 : wlo[c], r_hi = seg == 0 ? min(p.F, wlo[c]) : pos + 1;
+#pragma unroll
+              for (int t = 0; t < 2; ++t)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                  const int k = 16 * t + 4 * quad + r;
+                  const bool keep = kb + k >= r_lo && kb + k < min(r_hi, seg_hi) && ((bad >> k) & 1) == 0;
+                  c4[c][t][r] = keep ? c4[c][t][r] : -INFINITY;
+                }
+            }
           }
-        }
-        bf16x8_t pb[HPW], pl[HPW];
-#pragma unroll
-        for (int h = 0; h < HPW; ++h) {
-          // the softmax scale is applied inside exp2: m[h] is a raw score,
-          // p = 2^(q_scale (s - m))
-          float sv[8];
-#pragma unroll
-          for (int t = 0; t < 2; ++t)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) sv[4 * t + r] = c4[h][t][r];
           // lazy move of the reference point: p <= 2^8 stays exact in fp32.
           // The vote runs on each lane's own maximum (the four lanes of a
-          // row share m[h], so any lane exceeding it is the row maximum
-          // exceeding it): the row reduction is only needed when the point
-          // moves.  On the first block every present key moves it (acc and
-          // l are still zero, and the rescale by 2^(kNegBig - m_new) = 0
-          // leaves them zero).
-          float bmax = max8_nonan(sv);
-          const float vote = fresh ? -INFINITY : m[h] * p.q_scale + 8.0f;
-          if (__any(bmax * p.q_scale > vote)) {
-            bmax = quad_max(bmax);
-            const float m_new = max3_nonan(m[h], bmax, bmax);
-            const float alpha = fast_exp2((m[h] - m_new) * p.q_scale);
-            m[h] = m_new;
-            if (kRectify) l[h] *= alpha;
-            else l[h][0] *= alpha;
+          // column share m[c], so any lane exceeding it is the column's
+          // maximum exceeding it): the reduction over them is only needed
+          // when the point moves.  The first key a column sees moves it (acc
+          // and l are still zero, and the rescale by 2^(kNegBig - m_new) = 0
+          // leaves them zero).  The softmax scale is applied inside exp2:
+          // m[c] is a raw score, p = 2^(q_scale (s - m)).
+          float bmax[2];
 #pragma unroll
-            for (int dt = 0; dt < 8; ++dt) acc[h][dt] *= alpha;
+          for (int c = 0; c < 2; ++c) {
+            const float sv[8] = {c4[c][0][0], c4[c][0][1], c4[c][0][2], c4[c][0][3],
+                                 c4[c][1][0], c4[c][1][1], c4[c][1][2], c4[c][1][3]};
+            bmax[c] = max8_nonan(sv);
           }
-          const float mo = -m[h] * p.q_scale;
-          float psum = 0.0f;
+          if (__any(bmax[0] * p.q_scale > vt[0] || bmax[1] * p.q_scale > vt[1])) {
 #pragma unroll
-          for (int e = 0; e < 8; ++e) {
-            const float pe = fast_exp2(fmaf(sv[e], p.q_scale, mo));
-            if (!kRectify) psum = e == 0 ? pe : psum + pe;  // (0 + pe = pe: no add)
-            pb[h][e] = static_cast<__bf16>(pe);
-            // The fused form also feeds the bf16 rounding residual of P
-            // through a second MFMA (P = hi + lo, ~16 significant bits): the
-            // downdate divides the window's contribution by the prefix's
-            // share of the softmax mass, which amplifies any error of the
-            // window state.
-            if (kRectify) pl[h][e] = static_cast<__bf16>(pe - static_cast<float>(pb[h][e]));
+            for (int c = 0; c < 2; ++c) {
+              const float bm = quad_max(bmax[c]);
+              const float m_new = max3_nonan(m[c], bm, bm);
+              const float alpha = fast_exp2((m[c] - m_new) * p.q_scale);
+              m[c] = m_new;
+              vt[c] = m_new > kNegBig ? m_new * p.q_scale + 8.0f : -INFINITY;
+              if (kFused) l[c] *= alpha;
+              else l[c][0] *= alpha;
+#pragma unroll
+              for (int dt = 0; dt < 8; ++dt) acc[c][dt] *= alpha;
+            }
           }
-          if (!kRectify) l[h][0] += psum;
+          bf16x8_t pb[2], pl[2];
+#pragma unroll
+          for (int c = 0; c < 2; ++c) {
+            const float mo = -m[c] * p.q_scale;
+            float psum = 0.0f;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+              const float pe = fast_exp2(fmaf(c4[c][e >> 2][e & 3], p.q_scale, mo));
+              if (!kFused) psum = e == 0 ? pe : psum + pe;  // (0 + pe = pe: no add)
+              pb[c][e] = static_cast<__bf16>(pe);
+              // The fused form also feeds the bf16 rounding residual of P
+              // through a second MFMA (P = hi + lo, ~16 significant bits): the
+              // downdate divides the window's contribution by the prefix's
+              // share of the softmax mass, which amplifies any error of the
+              // window state.
+              if (kFused) pl[c][e] = static_cast<__bf16>(pe - static_cast<float>(pb[c][e]));
+            }
+            if (!kFused) l[c][0] += psum;
+          }
+          // O^T += V^T P^T (fused form: l += 1^T P^T as well)
+          if (kFused) {
+            const bf16x8_t ones = as_bf16x8(make_uint4(0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u));
+#pragma unroll
+            for (int c = 0; c < 2; ++c) {
+              l[c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, pb[c], l[c], 0, 0, 0);
+              l[c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, pl[c], l[c], 0, 0, 0);
+            }
+          }
+#pragma unroll
+          for (int dt = 0; dt < 8; ++dt)
+#pragma unroll
+            for (int c = 0; c < 2; ++c) {
+              acc[c][dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(va[dt], pb[c], acc[c][dt], 0, 0, 0);
+              if (kFused) acc[c][dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(va[dt], pl[c], acc[c][dt], 0, 0, 0);
+            }
         }
-        fresh = false;
-        // O^T += V^T P^T (fused form: l += 1^T P^T as well)
-        const bf16x8_t ones = as_bf16x8(make_uint4(0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u));
-#pragma unroll
-        for (int h = 0; h < HPW; ++h) {
-          if (kRectify) {
-            l[h] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, pb[h], l[h], 0, 0, 0);
-            l[h] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, pl[h], l[h], 0, 0, 0);
-          }
-        }
-#pragma unroll
-        for (int dt = 0; dt < 8; ++dt)
-#pragma unroll
-          for (int h = 0; h < HPW; ++h) {
-            acc[h][dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(va[dt], pb[h], acc[h][dt], 0, 0, 0);
-            if (kRectify) acc[h][dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(va[dt], pl[h], acc[h][dt], 0, 0, 0);
-          }
       }
       if (seg == 0) __syncthreads();  // the sink's last tiles are read before the window stages into them
     }
-    if (kRectify) {  // the rounds the blocks did not carry; then s_of is complete for every wave
+    if (kFused) {  // the rounds the blocks did not carry; then s_of is complete for every wave
       if (cq_pending) cq_store(cq - 1);
-      for (; cq < kHeadsPerTask; ++cq) {
+      for (; cq < kCq; ++cq) {
         cq_issue(cq);
         cq_store(cq);
       }
       __syncthreads();
     }
-    if (nheads == 0 || !row_ok) continue;
+    if (!live) continue;
 
-    if (!kRectify) {
+    if (kMode == kSplit && chunk < kNoChunk) {
+      // the piece's unnormalised state: O^T accumulators as the lanes hold
+      // them, and per column its reference point (log2 units) and sum
 #pragma unroll
-      for (int h = 0; h < HPW; ++h) {
-        if (h >= nheads) break;
-        const float lt = quad_sum(l[h][0]);
+      for (int c = 0; c < 2; ++c) {
+        const int64_t tile = static_cast<int64_t>(t) * kTiles + 2 * wave + c;
+        const float lt = quad_sum(l[c][0]);
+        f32x4_t* po = reinterpret_cast<f32x4_t*>(p.part_o) + tile * 8 * 64 + lane;
+        if (!row_ok[c]) continue;
+#pragma unroll
+        for (int dt = 0; dt < 8; ++dt) po[dt * 64] = acc[c][dt];
+        if (quad == 0) {
+          p.part_ml[(tile * 16 + col) * 2] = m[c] * p.q_scale;
+          p.part_ml[(tile * 16 + col) * 2 + 1] = lt;
+        }
+      }
+      continue;
+    }
+    if (!kFused) {
+#pragma unroll
+      for (int c = 0; c < 2; ++c) {
+        const float lt = quad_sum(l[c][0]);
+        if (!row_ok[c]) continue;
         const float inv = lt > 0.0f ? 1.0f / lt : 0.0f;
-        const int hq = hkv * G + hg0 + h;
-        uint16_t* op = p.out + (grow * Hq + hq) * kHeadDim + 4 * quad;
+        const int64_t at = (c == 0 ? grow0 : grow1) * Hq + hkv * G + hg0 + (c == 0 ? th0 : th1);
+        uint16_t* op = p.out + at * kHeadDim + 4 * quad;
 #pragma unroll
         for (int dt = 0; dt < 8; ++dt) {
           uint2 w;
-          w.x = pack2_bf16(acc[h][dt][0] * inv, acc[h][dt][1] * inv);
-          w.y = pack2_bf16(acc[h][dt][2] * inv, acc[h][dt][3] * inv);
+          w.x = pack2_bf16(acc[c][dt][0] * inv, acc[c][dt][1] * inv);
+          w.y = pack2_bf16(acc[c][dt][2] * inv, acc[c][dt][3] * inv);
           *reinterpret_cast<uint2*>(op + 16 * dt) = w;
         }
-        if (quad == 0) p.out_lse[grow * Hq + hq] = lt > 0.0f ? (m[h] * p.q_scale + fast_log2(lt)) * kLn2 : -INFINITY;
+        if (quad == 0) p.out_lse[at] = lt > 0.0f ? (m[c] * p.q_scale + fast_log2(lt)) * kLn2 : -INFINITY;
       }
       continue;
     }
@@ -753,56 +864,146 @@ __global__ void __launch_bounds__(256, (HPW == 1 && !kRectify) ? 3 : 2) window_k
     // ---- fused: downdate the full state, store the ring row ----
     if (req < 0 || req >= p.R) continue;
     if (before < 0) before = 0;
-    const int local = r_local + col;  // row index within the request
-    const int slot = static_cast<int>((static_cast<int64_t>(before) + local) % p.M);
-    const int64_t drow = static_cast<int64_t>(req) * p.M + slot;
-    const bool empty = pos + 1 - p.S <= (sink ? p.F : 0);  // nothing left after the downdate
-    // the full state's o of the lane's row, dims 16 dt + 4 quad .. + 3 of
-    // each of the wave's heads, from s_of
-    uint32_t fow[HPW][16];
     const uint2* of2 = reinterpret_cast<const uint2*>(s_of);
 #pragma unroll
-    for (int hh = 0; hh < HPW; ++hh) {
-#pragma unroll
-      for (int dt = 0; dt < 8; ++dt) {
-        const uint2 f = of2[2 * (col * kOfRow + 16 * (HPW * wave + hh) + 2 * dt + (quad >> 1)) + (quad & 1)];
-        fow[hh][2 * dt] = f.x;
-        fow[hh][2 * dt + 1] = f.y;
-      }
-    }
-#pragma unroll
-    for (int hh = 0; hh < HPW; ++hh) {
-      if (hh >= nheads) break;
-      const int h = hkv * G + hg0 + hh;
-      const float lt = l[hh][0];
+    for (int c = 0; c < 2; ++c) {
+      if (!row_ok[c]) continue;
+      const int local = r_local + row[c];  // row index within the request
+      const int slot = static_cast<int>((static_cast<int64_t>(before) + local) % p.M);
+      const int th = c == 0 ? th0 : th1;
+      const int64_t at = (static_cast<int64_t>(req) * p.M + slot) * Hq + hkv * G + hg0 + th;
+      const bool empty = pos0 + row[c] + 1 - p.S <= (sink ? p.F : 0);  // nothing left after the downdate
+      const float lt = l[c][0];
       const float inv = lt > 0.0f ? 1.0f / lt : 0.0f;
-      const float lse_w = lt > 0.0f ? (m[hh] * p.q_scale + fast_log2(lt)) * kLn2 : -INFINITY;
-      Downdate c;
+      const float lse_w = lt > 0.0f ? (m[c] * p.q_scale + fast_log2(lt)) * kLn2 : -INFINITY;
+      Downdate d;
       if (empty) {
-        c.lse = -INFINITY;
-        c.t = 0.0f;
-        c.scale = 0.0f;
+        d.lse = -INFINITY;
+        d.t = 0.0f;
+        d.scale = 0.0f;
       } else {
-        c = downdate_control(lse_full[hh], lse_w);
+        d = downdate_control(lse_full[c], lse_w);
       }
-      uint16_t* ap = p.attn_cache + (drow * Hq + h) * kHeadDim + 4 * quad;
+      // the full state's o of the lane's row, dims 16 dt + 4 quad .. + 3, from s_of
+      const int e = row[c] * kHeads + th;
+      const uint2* of = of2 + 2 * (16 * e + (e >> 2)) + quad;
+      uint16_t* ap = p.attn_cache + at * kHeadDim + 4 * quad;
 #pragma unroll
       for (int dt = 0; dt < 8; ++dt) {
+        const uint2 f = of[4 * dt];
+        const float fo[4] = {bf16_lo(f.x), bf16_hi(f.x), bf16_lo(f.y), bf16_hi(f.y)};
         float r[4];
-        const uint32_t fx = fow[hh][2 * dt], fy = fow[hh][2 * dt + 1];
-        const float fo[4] = {bf16_lo(fx), bf16_hi(fx), bf16_lo(fy), bf16_hi(fy)};
 #pragma unroll
-        for (int i = 0; i < 4; ++i) r[i] = empty ? 0.0f : (fo[i] - c.t * (acc[hh][dt][i] * inv)) * c.scale;
+        for (int i = 0; i < 4; ++i) r[i] = empty ? 0.0f : (fo[i] - d.t * (acc[c][dt][i] * inv)) * d.scale;
         uint2 w;
         w.x = pack2_bf16(r[0], r[1]);
         w.y = pack2_bf16(r[2], r[3]);
         *reinterpret_cast<uint2*>(ap + 16 * dt) = w;
       }
-      if (quad == 0) p.lse_cache[drow * Hq + h] = (p.sink_mode == 0 && p.F > 0) ? -INFINITY : c.lse;
+      if (quad == 0) p.lse_cache[at] = (p.sink_mode == 0 && p.F > 0) ? -INFINITY : d.lse;
       // (the pre-RoPE query row and the NaN marker of the unknown post-RoPE
       // row, PREFILL:251-262, went into the ring with the key blocks)
     }
   }
+}
+
+// Split form, second kernel: the states of a row block's pieces combined into
+// out and out_lse.  One workgroup per (row block, head chunk, column tile);
+// wave w sums the 16-dim tiles 2w, 2w + 1, lane for lane as window_kernel left
+// them, each piece weighted by 2^(m - max m), eight pieces' loads in flight (a
+// pass for the maxima first, one load at a time, took 70 of 206 us at one row
+// over 127K keys).  The workgroups past the batch's row blocks return.
+template <int RT>
+__global__ void __launch_bounds__(256) window_combine_kernel(WindowParams p) {
+  constexpr int kHeads = kTiles / RT;
+  constexpr int kRowsT = 16 * RT;
+  constexpr int kBatch = 8;
+  extern __shared__ int s_dyn[];
+  int* s_boff = s_dyn;               // [B + 1] pieces before a request
+  int* s_rows = s_dyn + (p.B + 1);   // [B + 1] row blocks before it
+  __shared__ int s_part[kWaves];
+  const int tid = threadIdx.x;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lane = tid & 63, quad = lane >> 4, col = lane & 15;
+  const int chunk = plan_pieces<kSplit, kRowsT>(p, s_boff, s_part);
+  if (chunk >= kNoChunk) return;  // window_kernel wrote the results
+  const int Hq = p.Hq, Hkv = p.Hkv, G = Hq / Hkv, B = p.B;
+  {
+    const int per = ceil_div(B, 256), b0 = min(B, tid * per), b1 = min(B, b0 + per);
+    int sum = 0, total;
+    for (int i = b0; i < b1; ++i) sum += ceil_div(request_rows<kSplit>(p, i), kRowsT);
+    int acc = scan256(sum, s_part, total);
+    for (int i = b0; i < b1; ++i) {
+      s_rows[i] = acc;
+      acc += ceil_div(request_rows<kSplit>(p, i), kRowsT);
+    }
+    if (tid == 0) s_rows[B] = total;
+    __syncthreads();
+  }
+  const int nchunks = ceil_div(G, kHeads);
+  const int per_piece = Hkv * nchunks;
+  const int tile = blockIdx.x % kTiles;
+  const int item = blockIdx.x / kTiles;
+  const int hc = item % per_piece;
+  const int rb = item / per_piece;  // row block, numbered over the batch
+  if (rb >= s_rows[B]) return;
+  const int b = request_of(s_rows, B, rb);
+  const int blk = rb - s_rows[b], nb = s_rows[b + 1] - s_rows[b];
+  const int q0 = p.qo_indptr[b];
+  const int len = p.qo_indptr[b + 1] - q0;
+  const int kvlen = p.kv_indptr[b + 1] - p.kv_indptr[b];
+  const int r_local = kRowsT * blk;
+  const int nrows = min(kRowsT, len - r_local);
+  const int pos_last = kvlen - len + r_local + nrows - 1;
+  const int hkv = hc / nchunks;
+  const int h = kHeads * (hc - hkv * nchunks) + tile / RT;  // head in the group
+  const int r0 = 16 * (tile % RT);
+  if (h >= G || r0 + col >= nrows) return;  // (window_kernel stored the lanes of whole rows only)
+  const int n = ceil_div(pos_last + 1, chunk);  // pieces with keys of these rows
+  auto slot = [&](int ch) {  // tile slot of chunk ch (window_kernel's task order)
+    return (static_cast<int64_t>(s_boff[b] + ch * nb + blk) * per_piece + hc) * kTiles + tile;
+  };
+  float mx = kNegBig, lt = 0.0f;
+  f32x4_t o[2] = {{0.0f, 0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f, 0.0f}};
+  for (int c0 = 0; c0 < n; c0 += kBatch) {
+    f32x4_t a[kBatch][2];
+    float w[kBatch], l[kBatch];
+#pragma unroll
+    for (int u = 0; u < kBatch; ++u) {
+      const int64_t t = slot(min(c0 + u, n - 1));
+      const f32x4_t* po = reinterpret_cast<const f32x4_t*>(p.part_o) + t * 8 * 64 + (2 * wave) * 64 + lane;
+      a[u][0] = po[0];
+      a[u][1] = po[64];
+      w[u] = p.part_ml[(t * 16 + col) * 2];
+      l[u] = p.part_ml[(t * 16 + col) * 2 + 1];
+    }
+    float m_new = mx;
+#pragma unroll
+    for (int u = 0; u < kBatch; ++u) m_new = fmaxf(m_new, w[u]);
+    const float keep = fast_exp2(mx - m_new);
+    mx = m_new;
+    lt *= keep;
+    o[0] *= keep;
+    o[1] *= keep;
+#pragma unroll
+    for (int u = 0; u < kBatch; ++u) {
+      const float f = c0 + u < n ? fast_exp2(w[u] - mx) : 0.0f;
+      lt += f * l[u];
+      o[0] += f * a[u][0];
+      o[1] += f * a[u][1];
+    }
+  }
+  const float inv = lt > 0.0f ? 1.0f / lt : 0.0f;
+  const int64_t at = (static_cast<int64_t>(q0) + r_local + r0 + col) * Hq + hkv * G + h;
+  uint16_t* op = p.out + at * kHeadDim + 4 * quad;
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    uint2 v;
+    v.x = pack2_bf16(o[i][0] * inv, o[i][1] * inv);
+    v.y = pack2_bf16(o[i][2] * inv, o[i][3] * inv);
+    *reinterpret_cast<uint2*>(op + 16 * (2 * wave + i)) = v;
+  }
+  if (quad == 0 && wave == 0) p.out_lse[at] = lt > 0.0f ? (mx + fast_log2(lt)) * kLn2 : -INFINITY;
 }
 
 // request_length[req] += len (indexed-by-request form, after the ring rows
@@ -836,20 +1037,87 @@ int grid_for(int64_t tasks, const void* kernel, size_t dyn_lds = 0) {
   return static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(wgs, static_cast<int64_t>(cus) * per_cu)));
 }
 
-// Launches the window kernel over `blocks` (a bound on the 16-row blocks of
-// the batch): two query heads per wave when the GQA group has more than four.
-template <bool kRectify>
-void launch_window(const WindowParams& p, int64_t blocks, hipStream_t stream) {
+// Row tiles of a task for a GQA group (window_kernel): 8 / RT heads cover it
+// without absent heads up to the next power of two.
+int row_tiles(int G) { return G > 4 ? 1 : (G > 2 ? 2 : (G > 1 ? 4 : 8)); }
+
+int device_cus() {
+  int dev = 0, v = 0;
+  if (hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || v <= 0)
+    return 256;
+  return v;
+}
+
+// Split over keys (causal attention over whole prefixes, window_left < 0):
+// pieces of the batch a split call plans for, or 0 where the row blocks alone
+// give the GPU enough work.  A task per (row block, head chunk) streams its
+// keys in one chain, so a batch with few of them leaves CUs idle; its keys
+// are then cut so that there are up to 1.5 rounds of the resident workgroups
+// (2 per CU) more tasks than row blocks.  Kept suffixes of long prompts are
+// that case: 512 rows over 32K keys, 4 heads per group, 839 -> 322 us
+// unsplit -> split; 8 requests of 16-32 rows over 8K-64K keys, 8 heads per
+// group, 1329 -> 196; one row over 127K keys 3340 -> 115.  One round more
+// instead took 318, 224 and 98 us, two 318, 196 and 134 (a piece's state is
+// 64 KiB written and read once), half a round 430 for the first.  From
+// 3/4 of a round of tasks on the cut costs what it levels out (32 requests x
+// 32 rows over 4K keys, 8 heads per group: 129 unsplit, 141 split), and below
+// kSplitKeys keys per request the second launch does (512 rows over 1024
+// keys: 34 and 36; 32 rows over 1024 keys: 33 and 25).
+constexpr int64_t kSplitKeys = 1024;
+struct Split {
+  int64_t blocks = 0;  // bound on the batch's row blocks
+  int pieces = 0;      // most (row block, key chunk) pieces; 0: no split
+  size_t o_bytes = 0, bytes = 0;
+};
+
+Split split_plan(int B, int Hq, int Hkv, int64_t total_q, int64_t kv_len, int window_left) {
+  Split sp;
+  if (window_left >= 0 || B <= 0 || total_q <= 0 || Hkv <= 0 || Hq < Hkv) return sp;
+  const int G = Hq / Hkv, rt = row_tiles(G);
+  const int64_t per_piece = static_cast<int64_t>(Hkv) * ceil_div(G, kTiles / rt);
+  // (a block holds at least one row, and every request but the first block of
+  // each fills its blocks)
+  sp.blocks = std::min<int64_t>(total_q, (total_q + 16 * rt - 1) / (16 * rt) + B);
+  const int64_t grid = 2 * static_cast<int64_t>(device_cus());
+  if (4 * sp.blocks * per_piece >= 3 * grid) return sp;
+  if (kv_len < kSplitKeys * static_cast<int64_t>(B)) return sp;
+  const int64_t pieces = sp.blocks + (3 * grid / 2 + per_piece - 1) / per_piece;
+  sp.pieces = static_cast<int>(pieces);
+  sp.o_bytes = static_cast<size_t>(pieces * per_piece) * kTiles * 8 * 64 * 16;
+  sp.bytes = sp.o_bytes + static_cast<size_t>(pieces * per_piece) * kTiles * 16 * 2 * sizeof(float);
+  return sp;
+}
+
+template <int RT>
+void launch_split(const WindowParams& p, const Split& sp, hipStream_t stream) {
+  const int64_t per_piece = static_cast<int64_t>(p.Hkv) * ceil_div(p.Hq / p.Hkv, kTiles / RT);
+  const size_t lds = sizeof(int) * (static_cast<size_t>(p.B) + 1);  // of one array over the requests
+  const void* kern = reinterpret_cast<const void*>(&window_kernel<RT, kSplit>);
+  hipLaunchKernelGGL((window_kernel<RT, kSplit>), dim3(grid_for(4 * sp.pieces * per_piece, kern, 3 * lds)), dim3(256),
+                     3 * lds, stream, p);
+  hipLaunchKernelGGL((window_combine_kernel<RT>), dim3(static_cast<unsigned>(sp.blocks * per_piece * kTiles)), dim3(256),
+                     2 * lds, stream, p);
+}
+
+template <int RT, int kMode>
+void launch_window_rt(const WindowParams& p, int64_t rows, hipStream_t stream) {
   const int G = p.Hq / p.Hkv;
   const size_t lds = 3 * sizeof(int) * (static_cast<size_t>(p.B) + 1);
-  if (G <= 4) {
-    const void* kern = reinterpret_cast<const void*>(&window_kernel<1, kRectify>);
-    hipLaunchKernelGGL((window_kernel<1, kRectify>), dim3(grid_for(4 * blocks * p.Hkv * ceil_div(G, 4), kern, lds)),
-                       dim3(256), lds, stream, p);
-  } else {
-    const void* kern = reinterpret_cast<const void*>(&window_kernel<2, kRectify>);
-    hipLaunchKernelGGL((window_kernel<2, kRectify>), dim3(grid_for(4 * blocks * p.Hkv * ceil_div(G, 8), kern, lds)),
-                       dim3(256), lds, stream, p);
+  const int64_t blocks = (rows + 16 * RT - 1) / (16 * RT) + p.B;  // (a bound)
+  const void* kern = reinterpret_cast<const void*>(&window_kernel<RT, kMode>);
+  const int64_t tasks = blocks * p.Hkv * ceil_div(G, kTiles / RT);
+  hipLaunchKernelGGL((window_kernel<RT, kMode>), dim3(grid_for(4 * tasks, kern, lds)), dim3(256), lds, stream, p);
+}
+
+// Launches the window kernel over at most `rows` query rows.
+template <int kMode>
+void launch_window(const WindowParams& p, int64_t rows, hipStream_t stream) {
+  switch (row_tiles(p.Hq / p.Hkv)) {
+    case 1: return launch_window_rt<1, kMode>(p, rows, stream);
+    case 2: return launch_window_rt<2, kMode>(p, rows, stream);
+    case 4: return launch_window_rt<4, kMode>(p, rows, stream);
+    default: return launch_window_rt<8, kMode>(p, rows, stream);
   }
 }
 
@@ -908,7 +1176,9 @@ int check_window_common(int B, int Hq, int Hkv, int D, int64_t total_q, int64_t 
 
 }  // namespace
 
-extern "C" int mac_prefill_window_attention_bf16(const MacWindowAttentionArgs* a, void* stream) {
+namespace {
+
+int check_window_args(const MacWindowAttentionArgs* a) {
   REQUIRE(a != nullptr, "args is NULL");
   REQUIRE(a->struct_size == sizeof(MacWindowAttentionArgs), "struct_size mismatch (%u vs %zu)", a->struct_size,
           sizeof(MacWindowAttentionArgs));
@@ -918,6 +1188,20 @@ extern "C" int mac_prefill_window_attention_bf16(const MacWindowAttentionArgs* a
     return rc;
   REQUIRE(a->out && a->out_lse, "out / out_lse must not be NULL");
   REQUIRE(aligned16(a->out), "out must be 16-byte aligned");
+  return MAC_OK;
+}
+
+}  // namespace
+
+extern "C" int64_t mac_prefill_window_attention_workspace(int32_t B, int32_t Hq, int32_t Hkv, int64_t total_q,
+                                                          int64_t kv_indices_len, int32_t window_left) {
+  return static_cast<int64_t>(split_plan(B, Hq, Hkv, total_q, kv_indices_len, window_left).bytes);
+}
+
+extern "C" int mac_prefill_window_attention_ws_bf16(const MacWindowAttentionArgs* a, void* workspace,
+                                                    int64_t workspace_bytes, void* stream) {
+  if (int rc = check_window_args(a)) return rc;
+  REQUIRE(workspace_bytes >= 0 && aligned16(workspace), "workspace must be 16-byte aligned");
   if (a->B == 0 || a->total_q == 0) return MAC_OK;
   WindowParams p{};
   p.q = static_cast<const uint16_t*>(a->q);
@@ -937,10 +1221,29 @@ extern "C" int mac_prefill_window_attention_bf16(const MacWindowAttentionArgs* a
   p.M = 1;
   p.window_left = a->window_left;
   p.q_scale = static_cast<float>(a->sm_scale * 1.4426950408889634);
-  const int64_t blocks = (a->total_q + kRows - 1) / kRows + a->B;
-  launch_window<false>(p, blocks, static_cast<hipStream_t>(stream));
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  const Split sp = workspace != nullptr
+                       ? split_plan(a->B, a->Hq, a->Hkv, a->total_q, a->kv_indices_len, a->window_left)
+                       : Split{};
+  if (sp.pieces > 0 && static_cast<int64_t>(sp.bytes) <= workspace_bytes) {
+    p.part_o = static_cast<float*>(workspace);
+    p.part_ml = reinterpret_cast<float*>(static_cast<char*>(workspace) + sp.o_bytes);
+    p.max_pieces = sp.pieces;
+    switch (row_tiles(p.Hq / p.Hkv)) {
+      case 1: launch_split<1>(p, sp, s); break;
+      case 2: launch_split<2>(p, sp, s); break;
+      case 4: launch_split<4>(p, sp, s); break;
+      default: launch_split<8>(p, sp, s); break;
+    }
+  } else {
+    launch_window<kPlain>(p, a->total_q, s);
+  }
   HIP_OK(hipGetLastError());
   return MAC_OK;
+}
+
+extern "C" int mac_prefill_window_attention_bf16(const MacWindowAttentionArgs* a, void* stream) {
+  return mac_prefill_window_attention_ws_bf16(a, nullptr, 0, stream);
 }
 
 extern "C" int mac_prefill_rectify_update_cache_bf16(const MacRectifyArgs* a, void* stream) {
@@ -995,9 +1298,8 @@ extern "C" int mac_prefill_rectify_update_cache_bf16(const MacRectifyArgs* a, vo
   p.rl_by_batch = a->request_length_len == a->B;
   p.q_scale = static_cast<float>(a->sm_scale * 1.4426950408889634);
   const int64_t kept = std::min<int64_t>(a->total_q, static_cast<int64_t>(a->B) * a->M);
-  const int64_t blocks = (kept + kRows - 1) / kRows + a->B;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  launch_window<true>(p, blocks, s);
+  launch_window<kRectify>(p, kept, s);
   HIP_OK(hipGetLastError());
   if (!p.rl_by_batch) {
     hipLaunchKernelGGL(bump_kernel, dim3((a->B + 255) / 256), dim3(256), 0, s, a->request_length, a->req_ids,

@@ -79,6 +79,8 @@ EXPORTED_SYMBOLS = (
     "mac_update_request_state",
     "mac_update_then_downdate_bf16_inplace",
     "mac_prefill_window_attention_bf16",
+    "mac_prefill_window_attention_ws_bf16",
+    "mac_prefill_window_attention_workspace",
     "mac_prefill_rectify_update_cache_bf16",
     "mac_decode_rope_preserve_q_bf16",
     "mac_last_error",
@@ -143,6 +145,10 @@ def load_library(path: str | None = None) -> ctypes.CDLL:
     lib.mac_update_then_downdate_bf16_inplace.restype = ctypes.c_int
     lib.mac_prefill_window_attention_bf16.argtypes = [ctypes.POINTER(MacWindowAttentionArgs), _p]
     lib.mac_prefill_window_attention_bf16.restype = ctypes.c_int
+    lib.mac_prefill_window_attention_ws_bf16.argtypes = [ctypes.POINTER(MacWindowAttentionArgs), _p, _i64, _p]
+    lib.mac_prefill_window_attention_ws_bf16.restype = ctypes.c_int
+    lib.mac_prefill_window_attention_workspace.argtypes = [_i32, _i32, _i32, _i64, _i64, _i32]
+    lib.mac_prefill_window_attention_workspace.restype = ctypes.c_int64
     lib.mac_prefill_rectify_update_cache_bf16.argtypes = [ctypes.POINTER(MacRectifyArgs), _p]
     lib.mac_prefill_rectify_update_cache_bf16.restype = ctypes.c_int
     lib.mac_decode_rope_preserve_q_bf16.argtypes = [
@@ -800,7 +806,13 @@ class PrefillRectifyExtension:
         a.B, a.Hq, a.Hkv, a.D = int(qo_indptr.shape[0]) - 1, hq, int(k_buffer.shape[1]), _HEAD_DIM
         a.window_left, a.sm_scale = int(window_left), float(sm_scale)
         with torch.cuda.device(q.device):
-            rc = self._lib.mac_prefill_window_attention_bf16(ctypes.byref(a), _stream(q.device))
+            # few rows over many keys: room for the partial states of a split
+            # over keys, from PyTorch's allocator (its stream-ordered reuse
+            # and graph pools keep it safe across streams and captures)
+            n = self._lib.mac_prefill_window_attention_workspace(a.B, a.Hq, a.Hkv, total_q, a.kv_indices_len,
+                                                                 a.window_left)
+            ws = torch.empty(n, device=q.device, dtype=torch.uint8) if n > 0 else None
+            rc = self._lib.mac_prefill_window_attention_ws_bf16(ctypes.byref(a), _ptr(ws), n, _stream(q.device))
         _raise_on(self._lib, rc)
         return out, out_lse
 

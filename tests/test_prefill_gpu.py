@@ -538,3 +538,95 @@ def test_window_attention_skips_requests_outside_the_buffers(rect_ext):
     assert rel_l2(got[:5], bits(eo[:5])) < 1e-2
     assert not got[5:].any() and (lse[5:] == 7.0).all()
     np.testing.assert_allclose(lse[:5].cpu().numpy(), el[:5], atol=2e-4)
+
+
+# ------------------------------------------- window attention split over keys ----
+
+
+def _unsplit(d, window_left, sm_scale, qo=None, kv=None):
+    """The same call without a workspace: one chain over a row block's keys."""
+    import ctypes
+
+    from mac_attention.integrations.sglang import bridge
+
+    lib = bridge.load_library()
+    qo, kv = d["qo"] if qo is None else qo, d["kv"] if kv is None else kv
+    out = torch.zeros_like(d["q"])
+    lse = torch.zeros(d["q"].shape[:2], device="cuda")
+    a = bridge.MacWindowAttentionArgs()
+    a.struct_size, a.abi_version = ctypes.sizeof(a), bridge.ABI_VERSION
+    a.q, a.k_buffer, a.v_buffer = d["q"].data_ptr(), d["k"].data_ptr(), d["v"].data_ptr()
+    a.qo_indptr, a.kv_indptr, a.kv_indices = qo.data_ptr(), kv.data_ptr(), d["idx"].data_ptr()
+    a.out, a.out_lse = out.data_ptr(), lse.data_ptr()
+    a.total_q, a.pool_tokens, a.kv_indices_len = d["q"].shape[0], d["k"].shape[0], d["idx"].shape[0]
+    a.B, a.Hq, a.Hkv, a.D = qo.shape[0] - 1, d["q"].shape[1], d["k"].shape[1], 128
+    a.window_left, a.sm_scale = window_left, sm_scale
+    assert lib.mac_prefill_window_attention_bf16(ctypes.byref(a), torch.cuda.current_stream().cuda_stream) == 0
+    torch.cuda.synchronize()
+    return out, lse
+
+
+def _workspace_bytes(d, window_left=-1, qo=None):
+    from mac_attention.integrations.sglang import bridge
+
+    qo = d["qo"] if qo is None else qo
+    return bridge.load_library().mac_prefill_window_attention_workspace(
+        qo.shape[0] - 1, d["q"].shape[1], d["k"].shape[1], d["q"].shape[0], d["idx"].shape[0], window_left)
+
+
+@pytest.mark.parametrize("hq,hkv", [(2, 2), (4, 2), (6, 2), (8, 2), (14, 2), (16, 2), (24, 2)])
+@pytest.mark.parametrize("qo_lens,kv_lens", [
+    ([1], [1024]),                            # one row, the shortest context that is split
+    ([16, 17], [4096, 1024 + 63]),            # a whole and a cut 16-row tile
+    ([31, 0, 129, 1], [2500, 40, 3000, 257]),  # an empty request, row blocks past a tile, a short context
+    ([1, 128], [9000, 129]),                  # most rows see a fraction of the chunks
+])
+def test_window_attention_split_over_keys(rect_ext, hq, hkv, qo_lens, kv_lens):
+    """Few rows over many keys: the keys of a row block are cut over several
+    workgroups and their states combined.  Every GQA tile shape (1, 2, 4, 8
+    row tiles, absent heads, two head chunks) against the oracle."""
+    print(f"split window: G={hq // hkv} qo={qo_lens} kv={kv_lens}", flush=True)
+    case = syn.prefill_case(qo_lens=qo_lens, kv_lens=kv_lens, hq=hq, hkv=hkv, seed=500 + hq)
+    d = _dev_case(case)
+    assert _workspace_bytes(d) > 0
+    out, lse = rect_ext.window_attention_return_lse(d["q"], d["k"], d["v"], d["qo"], d["kv"], d["idx"], -1,
+                                                    case.sm_scale)
+    torch.cuda.synchronize()
+    eo, el = orc.window_attention(_bf(case.q), _bf(case.k), _bf(case.v), case.qo_indptr, case.kv_indptr,
+                                  case.kv_indices, window_left=-1, sm_scale=case.sm_scale)
+    got = bits(_host_bits(out))
+    for r in range(got.shape[0]):
+        assert rel_l2(got[r], bits(eo[r])) < 1e-2, r
+    np.testing.assert_allclose(lse.cpu().numpy(), el, atol=2e-4, rtol=1e-5)
+
+
+def test_window_attention_split_keeps_bounds_and_masks(rect_ext):
+    """Split call, skipped and overlapping requests: rows of a request outside
+    the buffers stay untouched; keys without a pool row are masked; more row
+    blocks than the row count allows for (overlapping query ranges) give the
+    unsplit call's bits."""
+    case = syn.prefill_case(qo_lens=[20, 5], kv_lens=[3000, 2000], hq=8, hkv=2, seed=61)
+    d = _dev_case(case)
+    qo_bad = case.qo_indptr.copy()
+    qo_bad[2] = 5000
+    d["idx"][100:300] = -1
+    d["idx"][777] = d["k"].shape[0] + 5
+    assert _workspace_bytes(d) > 0
+    out = torch.zeros_like(d["q"])
+    lse = torch.full((25, 8), 7.0, device="cuda")
+    rect_ext.window_attention_return_lse(d["q"], d["k"], d["v"], _i32(qo_bad), d["kv"], d["idx"], -1, case.sm_scale,
+                                         out=out, out_lse=lse)
+    torch.cuda.synchronize()
+    uo, ul = _unsplit(d, -1, case.sm_scale)
+    assert rel_l2(bits(_host_bits(out))[:20], bits(_host_bits(uo))[:20]) < 5e-3
+    np.testing.assert_allclose(lse[:20].cpu().numpy(), ul[:20].cpu().numpy(), atol=2e-4)
+    assert not out[20:].any() and (lse[20:] == 7.0).all()
+    # 6 valid requests of the same 320 rows among 11: 120 row blocks, where the row count allows for 31
+    case = syn.prefill_case(qo_lens=[320], kv_lens=[12000], hq=96, hkv=12, seed=62)
+    d = _dev_case(case)
+    qo, kv = _i32(np.array([0, 320] * 6, np.int32)), _i32(np.array([0, 12000] * 6, np.int32))
+    assert _workspace_bytes(d, qo=qo) > 0
+    out, lse = rect_ext.window_attention_return_lse(d["q"], d["k"], d["v"], qo, kv, d["idx"], -1, case.sm_scale)
+    torch.cuda.synchronize()
+    uo, ul = _unsplit(d, -1, case.sm_scale, qo=qo, kv=kv)
+    assert torch.equal(out.view(torch.int16), uo.view(torch.int16)) and torch.equal(lse, ul)
