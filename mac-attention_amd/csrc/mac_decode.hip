@@ -5,8 +5,8 @@
 // allocation):
 //
 //  1. match_decide  (one workgroup per (request, KV head) group, four or
-//     eight waves; for rings of three or more 256-slot ranges, a range-split
-//     probe scan over (group, range) workgroups, then the decision kernel)
+//     eight waves; for rings of more than 128 slots, a range-split probe scan
+//     over (group, range) workgroups, then the decision kernel)
 //     Scans the request's ring of cached pre-RoPE queries for every query head
 //     of the group (squared L2, best = smallest distance, ties to the smaller
 //     logical position), applies the readiness gate and the optional synthetic
@@ -59,6 +59,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstdarg>
 #include <cstdio>
@@ -747,12 +748,14 @@ __device__ __forceinline__ uint32_t pack_bf16x2(float a, float b) {
 // group the scan of a large ring is bound by the loads each lane keeps in
 // flight.
 //
-// Large rings are scanned by a separate launch over (group, slot range)
-// (kMode 1, `splits` ranges of about kSplitSlots slots) that writes each
+// Larger rings are scanned by a separate launch over (group, slot range)
+// (kMode 1, `splits` ranges, scan_splits) that writes each
 // range's best into tile `range` of match_dist/pos/slot; match_decide then
 // reduces the tiles (kMode 2) instead of scanning.  kMode 0 scans and decides
 // in one workgroup per group.
 constexpr int kSplitSlots = 256;
+constexpr int kMinSplitSlots = 32;
+constexpr int kWholeRing = 128;
 // complete_task_go / _tile entries beyond 2 N Hkv: the long-group flag, one
 // spare, the previous step's counts for the short-group rule, one spare
 constexpr int kTaskExtra = 6;
@@ -803,19 +806,7 @@ __device__ __forceinline__ void decide_group(const DecideParams& p, const float 
     }
     return;
   }
-  if (kMode == 2) {  // best over the ranges' tiles
-    if (head_lane && eligible) {
-      for (int r = 0; r < p.splits; ++r) {
-        const float d = p.match_dist[mo + r];
-        const int ps = p.match_pos[mo + r];
-        if (p.match_slot[mo + r] >= 0 && better_pair(d, ps, bd, bp)) {
-          bd = d;
-          bp = ps;
-          bs = p.match_slot[mo + r];
-        }
-      }
-    }
-  } else if (head_lane) {
+  if (kMode == 0 && head_lane) {
     p.match_dist[mo] = bd;
     p.match_pos[mo] = bp;
     p.match_slot[mo] = bs;
@@ -1432,6 +1423,35 @@ __global__ void __launch_bounds__(W * 64, W == kWaves ? 2 : 1) match_decide_kern
       scan_batch(s_lo + wave);
     } else {
       for (int s0 = s_lo + wave; s0 < s_hi; s0 += W * kSlotBatch) scan_batch(s0);
+    }
+  }
+  if constexpr (kMode == 2) {
+    // best over the ranges' tiles: lane (row, c) of each wave takes every
+    // 16 W-th tile of its heads, the 16 lanes of a row then reduce (one lane
+    // per head reading tile after tile took 24 us at 128 ranges)
+#pragma unroll
+    for (int ps = 0; ps < kPasses; ++ps) {
+      const int hl = min(row + 4 * ps, G - 1);
+      const int64_t mo = (static_cast<int64_t>(n) * Hq + hkv * G + hl) * p.s.max_match_tiles;
+      for (int r = 16 * wave + c; r < p.splits; r += 16 * W) {
+        const float d = p.match_dist[mo + r];
+        const int pos = p.match_pos[mo + r], slot = p.match_slot[mo + r];
+        if (slot >= 0 && better_pair(d, pos, best_d[ps], best_p[ps])) {
+          best_d[ps] = d;
+          best_p[ps] = pos;
+          best_s[ps] = slot;
+        }
+      }
+#pragma unroll
+      for (int off = 1; off < 16; off <<= 1) {
+        const float od = __shfl_xor(best_d[ps], off);
+        const int op = __shfl_xor(best_p[ps], off), os = __shfl_xor(best_s[ps], off);
+        if (better_pair(od, op, best_d[ps], best_p[ps])) {
+          best_d[ps] = od;
+          best_p[ps] = op;
+          best_s[ps] = os;
+        }
+      }
     }
   }
 #pragma unroll
@@ -2326,6 +2346,22 @@ int fuse_tokens() {
   return x < 0 ? 0 : x;
 }
 
+// Slot ranges of the ring scan (1: match_decide scans the ring itself).
+// Rings of at most kWholeRing slots take the deciding workgroup one or two
+// rounds of loads; larger ones are scanned by a launch of their own, whose
+// probe reads half of most rows, in ranges of up to kSplitSlots slots, fewer
+// where the groups alone would leave CUs idle: two workgroups per CU, down to
+// kMinSplitSlots slots (one round of loads), as far as there are match tiles.
+// Step times (us) scanned in one workgroup / split, 4K contexts, hit 0.5, GQA-8:
+// 1 request, ring 128: 41.3 / 40.8, 192: 45.2 / 41.1, 512: 61.9 / 41.3; 16
+// requests, ring 512: 72 / 56; 64, ring 512: 123 / 113.  256-slot ranges alone
+// (rings of 513 slots on): 1 request, ring 2048: 57.6 / 42.5.
+int scan_splits(int M, int groups, int max_match_tiles, int cus) {
+  if (M <= kWholeRing) return 1;
+  const int most = std::min(max_match_tiles, ceil_div(M, kMinSplitSlots));
+  return std::max(1, std::min(most, std::max(ceil_div(M, kSplitSlots), ceil_div(2 * cus, groups))));
+}
+
 template <int G>
 void* attn_kernel_ptr() {
   return reinterpret_cast<void*>(&span_attention_mfma_kernel<G>);
@@ -2393,7 +2429,10 @@ int launch_all(const DecideParams& dp, const AttnParams& ap, const MergeParams& 
     MAC_HIP(hipGetLastError());
     DecideParams dp2 = dp;
     dp2.stamp_first = 0;  // the range scan recorded the step's start
-    hipLaunchKernelGGL((match_decide_kernel<G, 2>), dim3(NG), dim3(kBlock), 0, stream, dp2);
+    if (NG <= dp.fuse_cus && match_waves() == 8)
+      hipLaunchKernelGGL((match_decide_kernel<G, 2, 8>), dim3(NG), dim3(8 * 64), 0, stream, dp2);
+    else
+      hipLaunchKernelGGL((match_decide_kernel<G, 2>), dim3(NG), dim3(kBlock), 0, stream, dp2);
   } else if (NG <= dp.fuse_cus && match_waves() == 8) {
     // at most one group per CU: eight waves per group stream a finished
     // group's blocks in half the rounds
@@ -2529,11 +2568,10 @@ int mac::decode_impl(const MacDecodeArgs* a, void* stream_ptr, hipEvent_t* ev) {
   dp.group_tail_end = a->group_tail_end;
   dp.group_mode = a->group_mode;
   dp.task_counter = a->complete_task_tile + static_cast<int64_t>(N) * Hkv;
-  // rings of more than two ranges of kSplitSlots slots are scanned by a
-  // separate (group, range) launch, one match tile per range
-  dp.splits = std::max(1, std::min(a->max_match_tiles, ceil_div(M, kSplitSlots)));
+  // rings of more than kWholeRing slots are scanned by a separate (group,
+  // range) launch, one match tile per range
   dp.probe = match_probe();
-  if (dp.splits < 3) dp.splits = 1;
+  dp.splits = scan_splits(M, N * Hkv, a->max_match_tiles, cus);
   dp.S = a->semantic_pos_ahead;
   dp.F = a->front_sink_tokens > 0 ? a->front_sink_tokens : 0;
   dp.gen_min_limit = a->gen_min_limit;

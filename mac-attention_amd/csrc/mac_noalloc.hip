@@ -12,8 +12,8 @@
 // most kMaxHeads decode query heads (N * Hq), rings of at most
 // 256 * kMatchTiles slots, and kPartialSlots partial slots per group at that
 // many heads (the task plan enlarges a long group's chunks to fit them; a
-// step of fewer heads has the array's slots to itself, so that its groups
-// are cut as the workspace entry cuts them).  Every call on a
+// step of fewer heads has the array's slots and match tiles to itself, so
+// that its groups and rings are cut as the workspace entry cuts them).  Every call on a
 // device shares that device's array: calls that overlap on one GPU
 // (different streams) race.  Nothing in it needs clearing between calls:
 // the decode step's first kernel zeroes the task counter and rewrites every
@@ -134,9 +134,10 @@ extern "C" int mac_persistent_decode_bf16_noalloc(const MacDecodeArgs* a, void* 
   w.partial_lse = reinterpret_cast<float*>(base + L::partial_lse);
   w.partial_o = base + L::partial_o;
   w.partial_o_is_bf16 = 0;
-  w.max_match_tiles = kMatchTiles;
+  const int share = static_cast<int>(kMaxHeads / (heads > 0 ? heads : 1));  // of the array's tiles and slots
+  w.max_match_tiles = kMatchTiles * share;
   w.match_tile_slots = 256;
-  const int slots = kPartialSlots * static_cast<int>(kMaxHeads / (heads > 0 ? heads : 1));
+  const int slots = kPartialSlots * share;
   w.max_tiles_context = slots;
   w.tile_tokens = (a->max_context + slots - 1) / slots;
   w.complete_task_len = 2 * static_cast<int64_t>(a->N) * (a->Hkv > 0 ? a->Hkv : 1) + kTaskExtra;

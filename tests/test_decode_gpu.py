@@ -475,3 +475,26 @@ def test_small_step_chunks(partial, hkv, kv_lens, fuse, ext, monkeypatch):
         torch.cuda.synchronize()
         assert int(_np(w[22])[4]) == chunk, step
         _check_against_oracle(c, dev, out, out_lse, w, res, what=f"small step {step}")
+
+
+@pytest.mark.parametrize("ring,kv_lens,hkv", [
+    (128, [400, 90], 2),                 # the largest ring one workgroup scans
+    (129, [700, 100, 129, 130], 8),      # the smallest split one: five ranges, the last of one slot; unfilled rings
+    (300, [301, 5000], 4),               # a ring just full, and a wrapped one
+    (512, [2300, 511, 513], 1),
+    (4500, [6000, 4499], 2),             # more ranges than a row of lanes reads in one pass
+])
+@pytest.mark.parametrize("group", [1, 3, 4, 8])
+def test_split_ring_scan(ring, kv_lens, hkv, group, ext):
+    """Rings scanned in ranges by their own launch: range counts from the
+    ring, the groups and the match tiles; every decision against the oracle,
+    also with too few match tiles for the ranges the rule would take."""
+    print(f"split scan: ring={ring} kv={kv_lens} hkv={hkv} G={group}", flush=True)
+    c = syn.random_case(batch=len(kv_lens), hq=group * hkv, hkv=hkv, kv_lens=kv_lens, capacity=ring,
+                        semantic_pos_ahead=32, front_sink_tokens=8, hit_rate=0.6, match_lag=min(ring, 120) - 1, seed=ring)
+    res = oracle_run(c)
+    for tile_slots in (16, 256):
+        dev = syn.to_device(torch, c)
+        out, out_lse, ws = syn.run_decode(torch, ext, dev, c, max_context=6144, tile_tokens=32, match_tile_slots=tile_slots)
+        torch.cuda.synchronize()
+        _check_against_oracle(c, dev, out, out_lse, ws, res, what=f"split scan {ring} {tile_slots}")
