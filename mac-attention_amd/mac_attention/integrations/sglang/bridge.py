@@ -13,6 +13,7 @@ missing the loaders raise -- there is no fallback implementation.
 
 from __future__ import annotations
 
+import contextlib
 import ctypes
 import os
 from functools import lru_cache
@@ -215,7 +216,16 @@ def _check(cond: bool, msg: str) -> None:
         raise RuntimeError(msg)
 
 
+# A call checks some 40 tensors: one expression each when all is well, the
+# message's text only for a failed check.  (A direct decode step of one request
+# over a 4K context is bound by this host path: 46 us a call with four checks
+# and texts per tensor, a setattr per field and torch.cuda's device and stream
+# objects, 37 without; decode RoPE of 64 tokens 14.2 and 10.5.)
+
+
 def _check_tensor(t: torch.Tensor, name: str, dtype: torch.dtype, dim: int) -> None:
+    if t.is_cuda and t.dtype == dtype and t.dim() == dim and t.is_contiguous():
+        return
     _check(t.is_cuda, f"{name} must be CUDA")
     _check(t.is_contiguous(), f"{name} must be contiguous")
     _check(t.dtype == dtype, f"{name} has wrong dtype")
@@ -223,6 +233,8 @@ def _check_tensor(t: torch.Tensor, name: str, dtype: torch.dtype, dim: int) -> N
 
 
 def _check_partial_o(t: torch.Tensor, name: str) -> None:
+    if t.is_cuda and t.dtype in (torch.float32, torch.bfloat16) and t.dim() == 5 and t.is_contiguous():
+        return
     _check(t.is_cuda, f"{name} must be CUDA")
     _check(t.is_contiguous(), f"{name} must be contiguous")
     _check(t.dtype in (torch.float32, torch.bfloat16), f"{name} must be float32 or bfloat16")
@@ -239,8 +251,9 @@ def _env_flag(name: str, default: int) -> int:
         return 0
 
 
-# MacDecodeArgs fields of the 30 workspace tensors (prefixes)
-_WORKSPACE_FIELDS = ("match_", "head_", "group_", "complete_task_", "task_counts", "partial_")
+_DECODE_ARGS_SIZE = ctypes.sizeof(MacDecodeArgs)
+# the workspace pointers of MacDecodeArgs, for the no-allocation entry point
+_NO_WORKSPACES = (None,) * 21
 
 
 def _ptr(t: torch.Tensor | None) -> int | None:
@@ -250,7 +263,16 @@ def _ptr(t: torch.Tensor | None) -> int | None:
 
 
 def _stream(device: torch.device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    """The device's current stream, as torch.cuda.current_stream gives it."""
+    return torch._C._cuda_getCurrentRawStream(device.index)
+
+
+_NO_GUARD = contextlib.nullcontext()
+
+
+def _on_device(device: torch.device):
+    """torch.cuda.device(device), or nothing to do where it is current."""
+    return _NO_GUARD if torch._C._cuda_getDevice() == device.index else torch.cuda.device(device)
 
 
 class PersistentDecodeExtension:
@@ -268,7 +290,7 @@ class PersistentDecodeExtension:
         ``MAC_BENCH_EXACT_QUOTA`` are read from the environment on every call.
         """
         a, device = self._marshal(*args)
-        with torch.cuda.device(device):
+        with _on_device(device):
             rc = self._lib.mac_persistent_decode_bf16(ctypes.byref(a), _stream(device))
         _raise_on(self._lib, rc)
 
@@ -281,7 +303,7 @@ class PersistentDecodeExtension:
         and 2048 ring slots."""
         a, device = self._marshal(*args, use_workspaces=False)
         lib = load_noalloc_library()
-        with torch.cuda.device(device):
+        with _on_device(device):
             rc = lib.mac_persistent_decode_bf16_noalloc(ctypes.byref(a), _stream(device))
         if rc != 0:
             msg = lib.mac_noalloc_last_error().decode(errors="replace")
@@ -295,7 +317,7 @@ class PersistentDecodeExtension:
         a, device = self._marshal(*args)
         lib = load_bench_library()
         ms = (ctypes.c_float * 3)()
-        with torch.cuda.device(device):
+        with _on_device(device):
             rc = lib.mac_bench_decode_timed(ctypes.byref(a), _stream(device), ms)
         if rc != 0:
             raise RuntimeError(lib.mac_bench_last_error().decode(errors="replace") or f"code {rc}")
@@ -354,8 +376,9 @@ class PersistentDecodeExtension:
         _check_tensor(q_post, "q_post", bf16, 3)  # (the shape checks below read it)
         N, Hq, D = (int(x) for x in q_post.shape)
         Hkv = int(k_buffer.shape[1])
+        ws_rows = 0
         if use_workspaces:
-            self._check_workspaces(
+            ws_rows = self._check_workspaces(
                 N, Hq, Hkv, query_cache, max_context, tile_tokens, match_tile_slots, semantic_pos_ahead,
                 bench_mode, match_dist, match_pos, match_slot, head_hit, head_match_slot,
                 head_match_pos, head_prefix_end, head_rect_start, head_new_end, group_rect_begin,
@@ -366,21 +389,21 @@ class PersistentDecodeExtension:
         else:
             _check(int(bench_mode) in (0, 1, 2), "unsupported synthetic MAC bench mode")
         _check(D == _HEAD_DIM, "persistent decode v1 supports D=128 only")
-        _check(tuple(q_pre.shape) == tuple(q_post.shape), "q_pre/q_post shape mismatch")
-        _check(tuple(v_buffer.shape) == tuple(k_buffer.shape), "k/v shape mismatch")
+        _check(q_pre.shape == q_post.shape, "q_pre/q_post shape mismatch")
+        _check(v_buffer.shape == k_buffer.shape, "k/v shape mismatch")
         _check(int(k_buffer.shape[2]) == D, "k/v head_dim mismatch")
         _check(Hkv > 0 and Hq % Hkv == 0, "Hq must be divisible by Hkv")
         G = Hq // Hkv
         _check(0 < G <= _MAX_GROUP, "unsupported GQA group size")
         _check(req_ids.shape[0] >= N and past_lens.shape[0] >= N and out_cache_loc.shape[0] >= N,
                "batch metadata too small")
-        _check(tuple(out.shape) == tuple(q_post.shape), "out shape mismatch")
+        _check(out.shape == q_post.shape, "out shape mismatch")
         _check(optional_lse.numel() == 0 or optional_lse.numel() >= N * Hq,
                "optional_lse too small")
         R, M = int(query_cache.shape[0]), int(query_cache.shape[1])
         _check(query_cache.shape[2] == Hq and query_cache.shape[3] == D,
                "query_cache shape mismatch")
-        _check(tuple(attn_cache.shape) == tuple(query_cache.shape), "attn_cache shape mismatch")
+        _check(attn_cache.shape == query_cache.shape, "attn_cache shape mismatch")
         _check(tuple(lse_cache.shape) == (R, M, Hq), "lse_cache shape mismatch")
         return self._fill(
             N, Hq, Hkv, D, M, R, q_post, q_pre, k_buffer, v_buffer, req_to_token, req_ids, past_lens,
@@ -394,7 +417,7 @@ class PersistentDecodeExtension:
             gen_min_limit, lookback_right, candidate_mode, threshold, sm_scale, debug_enabled, bench_mode,
             bench_hit_rate, bench_hit_rate_std, bench_skip_ratio, bench_skip_ratio_std,
             bench_match_lag_mean, bench_match_lag_std, bench_seed, bench_miss_mask, bench_layer_id,
-            mac_cache_ready, mac_cache_epoch, mac_request_epoch, use_workspaces)
+            mac_cache_ready, mac_cache_epoch, mac_request_epoch, use_workspaces, ws_rows)
 
     @staticmethod
     def _check_workspaces(
@@ -405,9 +428,10 @@ class PersistentDecodeExtension:
         complete_task_go, complete_task_tile, tail_task_go, tail_task_tile, hit_tail_task_ho,
         hit_tail_task_tile, task_counts, partial_rect_o, partial_rect_lse, partial_rect_reduced_o,
         partial_rect_reduced_lse, partial_tail_o, partial_tail_lse,
-    ) -> None:
+    ) -> int:
         """The reference launcher's workspace checks (mac_decode_persistent.cu:5090-5153),
-        plus the complete-task minimum this build's kernels need."""
+        plus the complete-task minimum this build's kernels need.  Returns the
+        rows every head and group workspace has."""
         f32, i32 = torch.float32, torch.int32
         D = _HEAD_DIM
         G = Hq // Hkv if Hkv > 0 and Hq % Hkv == 0 else 1
@@ -457,13 +481,15 @@ class PersistentDecodeExtension:
         for name, t, tiles in (("rect output", partial_rect_o, mtc),
                                ("reduced rect output", partial_rect_reduced_o, mtr),
                                ("tail output", partial_tail_o, mtt)):
-            _check(t.shape[0] >= N and t.shape[1] == Hkv and t.shape[2] == tiles
-                   and t.shape[3] == G and t.shape[4] == D, f"{name} workspace has wrong shape")
+            n, *rest = t.shape
+            if n < N or rest != [Hkv, tiles, G, D]:
+                raise RuntimeError(f"{name} workspace has wrong shape")
         for name, t, tiles in (("rect lse", partial_rect_lse, mtc),
                                ("reduced rect lse", partial_rect_reduced_lse, mtr),
                                ("tail lse", partial_tail_lse, mtt)):
-            _check(t.shape[0] >= N and t.shape[1] == Hkv and t.shape[2] == tiles
-                   and t.shape[3] == G, f"{name} workspace has wrong shape")
+            n, *rest = t.shape
+            if n < N or rest != [Hkv, tiles, G]:
+                raise RuntimeError(f"{name} workspace has wrong shape")
         _check(group_mode.shape[0] >= N and group_mode.shape[1] >= Hkv,
                "group_mode workspace too small")
         _check(complete_task_tile.numel() == complete_task_go.numel(),
@@ -476,20 +502,21 @@ class PersistentDecodeExtension:
         _check(complete_task_go.numel() >= N * Hq * mtc, "complete task workspace too small")
         _check(tail_task_go.numel() >= N * Hkv * mtt, "tail task workspace too small")
         _check(hit_tail_task_ho.numel() >= N * Hq * mtt, "hit tail task workspace too small")
-        ws_rows = min(int(t.shape[0]) for t in (
-            head_hit, head_match_slot, head_match_pos, head_prefix_end, head_rect_start,
-            head_new_end, group_rect_begin, group_rect_end, group_rect_tiles, group_tail_begin,
-            group_tail_end, group_tail_tiles, group_mode, match_dist, match_pos, match_slot))
+        rows = []
         for t in (head_hit, head_match_slot, head_match_pos, head_prefix_end, head_rect_start,
                   head_new_end, match_dist, match_pos, match_slot):
-            _check(t.shape[1] == Hq, "head workspace must have Hq columns")
+            _check(t.size(1) == Hq, "head workspace must have Hq columns")
+            rows.append(t.size(0))
         for t in (group_rect_begin, group_rect_end, group_rect_tiles, group_tail_begin,
                   group_tail_end, group_tail_tiles, group_mode):
-            _check(t.shape[1] == Hkv, "group workspace must have Hkv columns")
+            _check(t.size(1) == Hkv, "group workspace must have Hkv columns")
+            rows.append(t.size(0))
+        ws_rows = min(rows)
         _check(ws_rows >= N, "head/group workspace has fewer rows than the batch")
         # this build's kernels keep per-group flags and the task counter there
         _check(complete_task_go.numel() >= 2 * N * Hkv + 6,
                "complete task workspace too small: needs at least 2 * N * Hkv + 6 entries")
+        return ws_rows
 
     @staticmethod
     def _fill(
@@ -504,7 +531,7 @@ class PersistentDecodeExtension:
         gen_min_limit, lookback_right, candidate_mode, threshold, sm_scale, debug_enabled, bench_mode,
         bench_hit_rate, bench_hit_rate_std, bench_skip_ratio, bench_skip_ratio_std,
         bench_match_lag_mean, bench_match_lag_std, bench_seed, bench_miss_mask, bench_layer_id,
-        mac_cache_ready, mac_cache_epoch, mac_request_epoch, use_workspaces,
+        mac_cache_ready, mac_cache_epoch, mac_request_epoch, use_workspaces, ws_rows,
     ) -> tuple[MacDecodeArgs, torch.device]:
         """The readiness-gate checks and the C argument block."""
         bf16, i64 = torch.bfloat16, torch.int64
@@ -524,67 +551,31 @@ class PersistentDecodeExtension:
                        "epoch tensors must cover every request slot")
                 epoch, req_epoch = mac_cache_epoch, mac_request_epoch
 
-        a = MacDecodeArgs()
-        a.struct_size = ctypes.sizeof(MacDecodeArgs)
-        a.abi_version = ABI_VERSION
-        for name, t in (("q_post", q_post), ("q_pre", q_pre), ("k_buffer", k_buffer),
-                        ("v_buffer", v_buffer), ("req_to_token", req_to_token),
-                        ("req_ids", req_ids), ("past_lens", past_lens),
-                        ("out_cache_loc", out_cache_loc), ("query_cache", query_cache),
-                        ("attn_cache", attn_cache), ("lse_cache", lse_cache), ("out", out),
-                        ("out_lse", optional_lse), ("match_dist", match_dist),
-                        ("match_pos", match_pos), ("match_slot", match_slot),
-                        ("head_hit", head_hit), ("head_match_slot", head_match_slot),
-                        ("head_match_pos", head_match_pos), ("head_prefix_end", head_prefix_end),
-                        ("head_rect_start", head_rect_start), ("head_new_end", head_new_end),
-                        ("group_rect_begin", group_rect_begin), ("group_rect_end", group_rect_end),
-                        ("group_rect_tiles", group_rect_tiles),
-                        ("group_tail_begin", group_tail_begin), ("group_tail_end", group_tail_end),
-                        ("group_tail_tiles", group_tail_tiles), ("group_mode", group_mode),
-                        ("complete_task_go", complete_task_go),
-                        ("complete_task_tile", complete_task_tile), ("task_counts", task_counts),
-                        ("partial_o", partial_rect_o), ("partial_lse", partial_rect_lse),
-                        ("cache_ready", ready), ("cache_epoch", epoch),
-                        ("request_epoch", req_epoch)):
-            if use_workspaces or not name.startswith(_WORKSPACE_FIELDS):
-                setattr(a, name, _ptr(t))
-        a.N, a.Hq, a.Hkv, a.D, a.M, a.R = N, Hq, Hkv, D, M, R
-        a.pool_tokens = int(k_buffer.shape[0])
-        a.req_to_token_rows = int(req_to_token.shape[0])
-        a.req_to_token_stride = int(req_to_token.shape[1])
-        a.out_cache_loc_is_i64 = 1 if out_cache_loc.dtype == i64 else 0
-        if use_workspaces:
-            a.max_match_tiles = int(match_dist.shape[2])
-            a.max_tiles_context = int(partial_rect_lse.shape[2])
-            a.partial_o_is_bf16 = 1 if partial_rect_o.dtype == bf16 else 0
-            a.complete_task_len = int(complete_task_go.numel())
-            a.workspace_rows = min(int(t.shape[0]) for t in (
-                head_hit, head_match_slot, head_match_pos, head_prefix_end, head_rect_start,
-                head_new_end, group_rect_begin, group_rect_end, group_rect_tiles, group_tail_begin,
-                group_tail_end, group_tail_tiles, group_mode, match_dist, match_pos, match_slot))
-        a.max_context = int(max_context)
-        a.tile_tokens = int(tile_tokens)
-        a.match_tile_slots = int(match_tile_slots)
-        a.semantic_pos_ahead = int(semantic_pos_ahead)
-        a.front_sink_tokens = int(front_sink_tokens)
-        a.gen_min_limit = int(gen_min_limit)
-        a.lookback_right = int(lookback_right)
-        a.candidate_mode = int(candidate_mode)
-        a.threshold = float(threshold)
-        a.sm_scale = float(sm_scale)
-        a.debug_enabled = int(debug_enabled)
-        a.bench_mode = int(bench_mode)
-        a.bench_hit_rate = float(bench_hit_rate)
-        a.bench_hit_rate_std = float(bench_hit_rate_std)
-        a.bench_skip_ratio = float(bench_skip_ratio)
-        a.bench_skip_ratio_std = float(bench_skip_ratio_std)
-        a.bench_match_lag_mean = float(bench_match_lag_mean)
-        a.bench_match_lag_std = float(bench_match_lag_std)
-        a.bench_seed = int(bench_seed)
-        a.bench_miss_mask = int(bench_miss_mask)
-        a.bench_layer_id = int(bench_layer_id)
-        a.mixed_group_fallback = _env_flag("MAC_PERSISTENT_MIXED_GROUP_FALLBACK", 1)
-        a.bench_exact_quota = _env_flag("MAC_BENCH_EXACT_QUOTA", 1)
+        w = use_workspaces
+        a = MacDecodeArgs(  # in field order
+            _DECODE_ARGS_SIZE, ABI_VERSION,
+            _ptr(q_post), _ptr(q_pre), _ptr(k_buffer), _ptr(v_buffer), _ptr(req_to_token), _ptr(req_ids),
+            _ptr(past_lens), _ptr(out_cache_loc), _ptr(query_cache), _ptr(attn_cache), _ptr(lse_cache),
+            _ptr(out), _ptr(optional_lse),
+            *((_ptr(match_dist), _ptr(match_pos), _ptr(match_slot),
+               _ptr(head_hit), _ptr(head_match_slot), _ptr(head_match_pos),
+               _ptr(head_prefix_end), _ptr(head_rect_start), _ptr(head_new_end),
+               _ptr(group_rect_begin), _ptr(group_rect_end), _ptr(group_rect_tiles),
+               _ptr(group_tail_begin), _ptr(group_tail_end), _ptr(group_tail_tiles),
+               _ptr(group_mode), _ptr(complete_task_go), _ptr(complete_task_tile), _ptr(task_counts),
+               _ptr(partial_rect_o), _ptr(partial_rect_lse)) if w else _NO_WORKSPACES),
+            _ptr(ready), _ptr(epoch), _ptr(req_epoch),
+            N, Hq, Hkv, D, M, R, k_buffer.size(0), req_to_token.size(0), req_to_token.size(1),
+            1 if out_cache_loc.dtype == i64 else 0,
+            *((match_dist.size(2), partial_rect_lse.size(2), 1 if partial_rect_o.dtype == bf16 else 0,
+               complete_task_go.numel(), ws_rows) if w else (0, 0, 0, 0, 0)),
+            int(max_context), int(tile_tokens), int(match_tile_slots), int(semantic_pos_ahead),
+            int(front_sink_tokens), int(gen_min_limit), int(lookback_right), int(candidate_mode),
+            float(threshold), float(sm_scale), int(debug_enabled), int(bench_mode),
+            float(bench_hit_rate), float(bench_hit_rate_std), float(bench_skip_ratio),
+            float(bench_skip_ratio_std), float(bench_match_lag_mean), float(bench_match_lag_std),
+            int(bench_seed), int(bench_miss_mask), int(bench_layer_id),
+            _env_flag("MAC_PERSISTENT_MIXED_GROUP_FALLBACK", 1), _env_flag("MAC_BENCH_EXACT_QUOTA", 1))
         if phase_cycles is not None:
             a.phase_cycles = _ptr(phase_cycles)
             a.phase_cycles_len = int(phase_cycles.numel())
@@ -612,9 +603,10 @@ class PrefillUpdateCacheExtension:
                             ("offsets", offsets, torch.int32), ("src_q", src_q, torch.bfloat16),
                             ("src_attn", src_attn, torch.bfloat16),
                             ("src_lse", src_lse, torch.float32)):
-            _check(t.is_cuda, f"{name} must be a CUDA tensor")
-            _check(t.is_contiguous(), f"{name} must be contiguous")
-            _check(t.dtype == dt, f"{name} has wrong dtype")
+            if not (t.is_cuda and t.dtype == dt and t.is_contiguous()):
+                _check(t.is_cuda, f"{name} must be a CUDA tensor")
+                _check(t.is_contiguous(), f"{name} must be contiguous")
+                _check(t.dtype == dt, f"{name} has wrong dtype")
         R = int(q_cache.shape[0])
         _check(R > 0, "R must be > 0")
         _check(q_cache.dim() == 4, "q_cache must be [R,M,H,D]")
@@ -641,7 +633,7 @@ class PrefillUpdateCacheExtension:
             _check(tuple(q_post_cache.shape) == tuple(q_cache.shape),
                    "q_post_cache must match q_cache")
             qpc = q_post_cache
-        with torch.cuda.device(q_cache.device):
+        with _on_device(q_cache.device):
             rc = self._lib.mac_prefill_update_cache(
                 _ptr(q_cache), _ptr(attn_cache), _ptr(lse_cache), _ptr(request_length),
                 int(request_length.shape[0]), _ptr(req_ids), B, _ptr(src_q), _ptr(src_attn),
@@ -656,9 +648,10 @@ class PrefillUpdateCacheExtension:
         for name, t, dt in (("cache_epoch", cache_epoch, torch.int64),
                             ("request_epoch", request_epoch, torch.int64),
                             ("req_ids", req_ids, torch.int32)):
-            _check(t.is_cuda, f"{name} must be a CUDA tensor")
-            _check(t.is_contiguous(), f"{name} must be contiguous")
-            _check(t.dtype == dt, f"{name} has wrong dtype")
+            if not (t.is_cuda and t.dtype == dt and t.is_contiguous()):
+                _check(t.is_cuda, f"{name} must be a CUDA tensor")
+                _check(t.is_contiguous(), f"{name} must be contiguous")
+                _check(t.dtype == dt, f"{name} has wrong dtype")
         _check(cache_epoch.shape[0] == ready.shape[0], "cache_epoch must match ready")
         _check(request_epoch.shape[0] == ready.shape[0], "request_epoch must match ready")
 
@@ -666,7 +659,7 @@ class PrefillUpdateCacheExtension:
         if req_ids.shape[0] == 0:
             return
         self._ready_common(ready, cache_epoch, request_epoch, req_ids)
-        with torch.cuda.device(ready.device):
+        with _on_device(ready.device):
             rc = self._lib.mac_mark_persistent_ready(
                 _ptr(ready), _ptr(cache_epoch), _ptr(request_epoch), _ptr(req_ids),
                 int(req_ids.shape[0]), int(ready.shape[0]), _stream(ready.device))
@@ -676,7 +669,7 @@ class PrefillUpdateCacheExtension:
         if req_ids.shape[0] == 0:
             return
         self._ready_common(ready, cache_epoch, request_epoch, req_ids)
-        with torch.cuda.device(ready.device):
+        with _on_device(ready.device):
             rc = self._lib.mac_invalidate_persistent_ready(
                 _ptr(ready), _ptr(cache_epoch), _ptr(request_epoch), _ptr(req_ids),
                 int(req_ids.shape[0]), int(ready.shape[0]), _stream(ready.device))
@@ -689,15 +682,16 @@ class PrefillUpdateCacheExtension:
         for name, t in (("req_len", req_len), ("match_req_len", match_req_len),
                         ("cache_lens", cache_lens), ("req_ids", req_ids), ("seq_lens", seq_lens),
                         ("cur_lens", cur_lens)):
-            _check(t.is_cuda, f"{name} must be a CUDA tensor")
-            _check(t.is_contiguous(), f"{name} must be contiguous")
-            _check(t.dtype == torch.int32, f"{name} has wrong dtype")
+            if not (t.is_cuda and t.dtype == torch.int32 and t.is_contiguous()):
+                _check(t.is_cuda, f"{name} must be a CUDA tensor")
+                _check(t.is_contiguous(), f"{name} must be contiguous")
+                _check(t.dtype == torch.int32, f"{name} has wrong dtype")
         B = int(req_ids.shape[0])
         _check(match_req_len.shape[0] == req_len.shape[0], "match_req_len must match req_len")
         _check(seq_lens.shape[0] >= B, "seq_lens is shorter than req_ids")
         _check(cur_lens.shape[0] >= B, "cur_lens is shorter than req_ids")
         _check(cache_lens.shape[0] >= B, "cache_lens is shorter than req_ids")
-        with torch.cuda.device(req_len.device):
+        with _on_device(req_len.device):
             rc = self._lib.mac_update_request_state(
                 _ptr(req_len), _ptr(match_req_len), _ptr(cache_lens), _ptr(req_ids),
                 _ptr(seq_lens), _ptr(cur_lens), B, int(req_len.shape[0]), _stream(req_len.device))
@@ -751,7 +745,7 @@ class MergeDowndateExtension:
                    f"{name} must be float32, bfloat16, or float16; got {t.dtype}")
         n, h, d = (int(x) for x in out1_bf16.shape)
         _check(tuple(lse1_any.shape) == (n, h), "lse1 must be [N,H]")
-        with torch.cuda.device(out1_bf16.device):
+        with _on_device(out1_bf16.device):
             rc = self._lib.mac_update_then_downdate_bf16_inplace(
                 _ptr(out1_bf16), _ptr(lse1_any), _LSE_DTYPES[lse1_any.dtype], _ptr(out2_bf16),
                 _ptr(lse2_any), _LSE_DTYPES[lse2_any.dtype], n * h, d, _stream(out1_bf16.device))
@@ -762,9 +756,10 @@ def _check_ragged(q, k_buffer, v_buffer, qo_indptr, kv_indptr, kv_indices):
     for name, t, dt in (("q", q, torch.bfloat16), ("k_buffer", k_buffer, torch.bfloat16),
                         ("v_buffer", v_buffer, torch.bfloat16), ("qo_indptr", qo_indptr, torch.int32),
                         ("kv_indptr", kv_indptr, torch.int32), ("kv_indices", kv_indices, torch.int32)):
-        _check(t.is_cuda, f"{name} must be CUDA")
-        _check(t.is_contiguous(), f"{name} must be contiguous")
-        _check(t.dtype == dt, f"{name} has wrong dtype")
+        if not (t.is_cuda and t.dtype == dt and t.is_contiguous()):
+            _check(t.is_cuda, f"{name} must be CUDA")
+            _check(t.is_contiguous(), f"{name} must be contiguous")
+            _check(t.dtype == dt, f"{name} has wrong dtype")
     _check(q.dim() == 3 and int(q.shape[2]) == _HEAD_DIM, "q must be [total_q,Hq,128]")
     _check(k_buffer.dim() == 3 and k_buffer.shape == v_buffer.shape, "k/v buffers must be [pool,Hkv,128]")
     _check(int(k_buffer.shape[2]) == _HEAD_DIM, "k/v head_dim mismatch")
@@ -805,7 +800,7 @@ class PrefillRectifyExtension:
         a.kv_indices_len = int(kv_indices.shape[0])
         a.B, a.Hq, a.Hkv, a.D = int(qo_indptr.shape[0]) - 1, hq, int(k_buffer.shape[1]), _HEAD_DIM
         a.window_left, a.sm_scale = int(window_left), float(sm_scale)
-        with torch.cuda.device(q.device):
+        with _on_device(q.device):
             # few rows over many keys: room for the partial states of a split
             # over keys, from PyTorch's allocator (its stream-ordered reuse
             # and graph pools keep it safe across streams and captures)
@@ -828,9 +823,10 @@ class PrefillRectifyExtension:
                             ("lse_cache", lse_cache, torch.float32),
                             ("request_length", request_length, torch.int32),
                             ("req_ids", req_ids, torch.int32)):
-            _check(t.is_cuda, f"{name} must be a CUDA tensor")
-            _check(t.is_contiguous(), f"{name} must be contiguous")
-            _check(t.dtype == dt, f"{name} has wrong dtype")
+            if not (t.is_cuda and t.dtype == dt and t.is_contiguous()):
+                _check(t.is_cuda, f"{name} must be a CUDA tensor")
+                _check(t.is_contiguous(), f"{name} must be contiguous")
+                _check(t.dtype == dt, f"{name} has wrong dtype")
         _check(src_q.shape == q_post.shape and o_full.shape == q_post.shape,
                "src_q / o_full must match q_post [total_q,Hq,128]")
         total_q, hq, _ = (int(x) for x in q_post.shape)
@@ -864,7 +860,7 @@ class PrefillRectifyExtension:
         a.B, a.R, a.M, a.Hq, a.Hkv, a.D = B, R, M, hq, int(k_buffer.shape[1]), _HEAD_DIM
         a.semantic_pos_ahead, a.front_sink_tokens = int(semantic_pos_ahead), int(front_sink_tokens)
         a.sink_mode, a.sm_scale = int(sink_mode), float(sm_scale)
-        with torch.cuda.device(q_post.device):
+        with _on_device(q_post.device):
             rc = self._lib.mac_prefill_rectify_update_cache_bf16(ctypes.byref(a), _stream(q_post.device))
         _raise_on(self._lib, rc)
 
@@ -896,15 +892,17 @@ class DecodeRopePreserveExtension:
                                         positions, cache_locs, head_dim: int, is_neox: bool) -> None:
         """Checks and messages of mac_decode_rope_preserve.cu:158-221."""
         for name, t in (("q", q), ("k", k), ("v", v)):
-            _check(t.is_cuda, f"{name} must be CUDA")
-            _check(t.dtype == torch.bfloat16, f"{name} has wrong dtype")
-            _check(t.dim() == 2, f"{name} must have rank 2")
-            _check(t.stride(1) == 1, f"{name} must have contiguous last dimension")
+            if not (t.is_cuda and t.dtype == torch.bfloat16 and t.dim() == 2 and t.stride(1) == 1):
+                _check(t.is_cuda, f"{name} must be CUDA")
+                _check(t.dtype == torch.bfloat16, f"{name} has wrong dtype")
+                _check(t.dim() == 2, f"{name} must have rank 2")
+                _check(t.stride(1) == 1, f"{name} must have contiguous last dimension")
         for name, t in (("q_pre", q_pre), ("k_buffer", k_buffer), ("v_buffer", v_buffer)):
-            _check(t.is_cuda, f"{name} must be CUDA")
-            _check(t.dtype == torch.bfloat16, f"{name} has wrong dtype")
-            _check(t.dim() == 3, f"{name} must have rank 3")
-            _check(t.is_contiguous(), f"{name} must be contiguous")
+            if not (t.is_cuda and t.dtype == torch.bfloat16 and t.dim() == 3 and t.is_contiguous()):
+                _check(t.is_cuda, f"{name} must be CUDA")
+                _check(t.dtype == torch.bfloat16, f"{name} has wrong dtype")
+                _check(t.dim() == 3, f"{name} must have rank 3")
+                _check(t.is_contiguous(), f"{name} must be contiguous")
         _check(cos_sin_cache.is_cuda, "cos_sin_cache must be CUDA")
         _check(cos_sin_cache.dtype == torch.float32, "cos_sin_cache has wrong dtype")
         _check(cos_sin_cache.dim() == 2, "cos_sin_cache must have rank 2")
@@ -934,7 +932,7 @@ class DecodeRopePreserveExtension:
         _check(0 < rot <= head_dim and rot % 2 == 0, "invalid rotary_dim")
         if n == 0:
             return
-        with torch.cuda.device(q.device):
+        with _on_device(q.device):
             rc = self._lib.mac_decode_rope_preserve_q_bf16(
                 _ptr(q), int(q.stride(0)), _ptr(k), int(k.stride(0)), _ptr(v), int(v.stride(0)),
                 _ptr(q_pre), int(q_pre.shape[0]), _ptr(k_buffer), _ptr(v_buffer), int(k_buffer.shape[0]),
