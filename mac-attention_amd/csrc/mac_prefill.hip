@@ -1053,13 +1053,15 @@ int device_cus() {
 // pieces of the batch a split call plans for, or 0 where the row blocks alone
 // give the GPU enough work.  A task per (row block, head chunk) streams its
 // keys in one chain, so a batch with few of them leaves CUs idle; its keys
-// are then cut so that there are up to 1.5 rounds of the resident workgroups
+// are then cut so that there are up to two rounds of the resident workgroups
 // (2 per CU) more tasks than row blocks.  Kept suffixes of long prompts are
-// that case: 512 rows over 32K keys, 4 heads per group, 839 -> 322 us
+// that case: 512 rows over 32K keys, 4 heads per group, 839 -> 318 us
 // unsplit -> split; 8 requests of 16-32 rows over 8K-64K keys, 8 heads per
-// group, 1329 -> 196; one row over 127K keys 3340 -> 115.  One round more
-// instead took 318, 224 and 98 us, two 318, 196 and 134 (a piece's state is
-// 64 KiB written and read once), half a round 430 for the first.  From
+// group, 1329 -> 196; one row over 127K keys 3340 -> 134.  One round more
+// instead took 318, 224 and 98 us (no second round to level the ragged
+// batch), 1.5 rounds 323, 196 and 115 (a half-empty last round for the even
+// one), three 328, 194 and 167 (a piece's state is 64 KiB written and read
+// once), half a round 430 for the first.  From
 // 3/4 of a round of tasks on the cut costs what it levels out (32 requests x
 // 32 rows over 4K keys, 8 heads per group: 129 unsplit, 141 split), and below
 // kSplitKeys keys per request the second launch does (512 rows over 1024
@@ -1082,7 +1084,7 @@ Split split_plan(int B, int Hq, int Hkv, int64_t total_q, int64_t kv_len, int wi
   const int64_t grid = 2 * static_cast<int64_t>(device_cus());
   if (4 * sp.blocks * per_piece >= 3 * grid) return sp;
   if (kv_len < kSplitKeys * static_cast<int64_t>(B)) return sp;
-  const int64_t pieces = sp.blocks + (3 * grid / 2 + per_piece - 1) / per_piece;
+  const int64_t pieces = sp.blocks + (2 * grid + per_piece - 1) / per_piece;
   sp.pieces = static_cast<int>(pieces);
   sp.o_bytes = static_cast<size_t>(pieces * per_piece) * kTiles * 8 * 64 * 16;
   sp.bytes = sp.o_bytes + static_cast<size_t>(pieces * per_piece) * kTiles * 16 * 2 * sizeof(float);
