@@ -10,9 +10,9 @@
 //
 //  * downdate_kernel: the reference's downdate op on its own (any head_dim,
 //    f32/bf16/f16 lse), for callers that keep the reference's three calls.
-//  * window_kernel<RT, kPlain>: causal sliding-window attention over a
+//  * window_kernel<RT, kPlain, ..>: causal sliding-window attention over a
 //    ragged batch with a page-size-1 KV pool (the windowed FlashInfer pass).
-//  * window_kernel<RT, kRectify>: the fused form.  Only the rows the ring keeps
+//  * window_kernel<RT, kRectify, ..>: the fused form.  Only the rows the ring keeps
 //    (the last min(len, M) of each request) are computed; for them the window
 //    state never leaves registers: it is downdated from the full state and
 //    stored straight into the ring with the pre-RoPE query, followed by the
@@ -334,9 +334,9 @@ __device__ __forceinline__ int request_of(const int* s_boff, int B, int piece) {
 // 4: 16 rows x 8 heads; 3, 4: 32 x 4; 2: 64 x 2; 1: 128 x 1).  Each of the
 // four waves owns two of them, so every K and V operand a wave reads from LDS
 // feeds 32 columns whatever the group size.  K/V rows are staged in
-// double-buffered LDS tiles of kBlk keys: 64 (plain; one barrier and one
-// round of address work per 64 keys), or 32 (fused form, whose epilogue also
-// holds the full state's rows in LDS).  Per wave and 32 keys:
+// double-buffered LDS tiles of kBlk keys: 64 (one barrier and one round of
+// address work per 64 keys), or 32 (fused form, whose epilogue also holds the
+// full state's rows in LDS, and far windows, see launch_window_rt).  Per wave and 32 keys:
 //  * S^T = K Q^T: the A operand of score tile t, row m, is key 16 t + m; the
 //    lane holding column col ends up with the scores of keys 16 t + 4 quad +
 //    (0..3), quad = lane / 16.
@@ -368,12 +368,12 @@ __device__ __forceinline__ int request_of(const int* s_boff, int B, int piece) {
 constexpr int kKRow = 16;  // 16-byte units per staged K row
 constexpr int kVRow = 18;  // per staged V row: 256 + 32
 
-template <int RT, int kMode>
+template <int RT, int kMode, int kBlk>
 __global__ void __launch_bounds__(256, 2) window_kernel(WindowParams p) {
   constexpr bool kFused = kMode == kRectify;
   constexpr int kHeads = kTiles / RT;   // query heads of a task
   constexpr int kRowsT = 16 * RT;       // query rows of a task
-  constexpr int kBlk = kFused ? 32 : 64;  // keys per staged block
+  constexpr bool kFarWindow = kMode == kPlain && kBlk == 32;  // (launch_window_rt)
   constexpr int kSub = kBlk / 32;
   constexpr int kLd = kBlk / 16;  // keys each thread stages a chunk of
   // dynamic: s_boff[B + 1] piece offsets, s_qo[B + 1] / s_kv[B + 1] the
@@ -607,6 +607,7 @@ __global__ void __launch_bounds__(256, 2) window_kernel(WindowParams p) {
       ok = 0;
 #pragma unroll
       for (int i = 0; i < kLd; ++i) {
+        if (kFarWindow && base + 16 * i >= end) continue;  // (uniform: none of these 16 keys exists)
         const bool in = base + ld_key + 16 * i < end && static_cast<unsigned>(raw[i]) < pool_rows;
         ok |= in ? 1u << i : 0u;
         const char* at = kbase + static_cast<uint64_t>(static_cast<uint32_t>(in ? raw[i] : 0)) * row_bytes;
@@ -1095,21 +1096,42 @@ template <int RT>
 void launch_split(const WindowParams& p, const Split& sp, hipStream_t stream) {
   const int64_t per_piece = static_cast<int64_t>(p.Hkv) * ceil_div(p.Hq / p.Hkv, kTiles / RT);
   const size_t lds = sizeof(int) * (static_cast<size_t>(p.B) + 1);  // of one array over the requests
-  const void* kern = reinterpret_cast<const void*>(&window_kernel<RT, kSplit>);
-  hipLaunchKernelGGL((window_kernel<RT, kSplit>), dim3(grid_for(4 * sp.pieces * per_piece, kern, 3 * lds)), dim3(256),
+  const void* kern = reinterpret_cast<const void*>(&window_kernel<RT, kSplit, 64>);
+  hipLaunchKernelGGL((window_kernel<RT, kSplit, 64>), dim3(grid_for(4 * sp.pieces * per_piece, kern, 3 * lds)), dim3(256),
                      3 * lds, stream, p);
   hipLaunchKernelGGL((window_combine_kernel<RT>), dim3(static_cast<unsigned>(sp.blocks * per_piece * kTiles)), dim3(256),
                      2 * lds, stream, p);
 }
 
-template <int RT, int kMode>
-void launch_window_rt(const WindowParams& p, int64_t rows, hipStream_t stream) {
+template <int RT, int kMode, int kBlk>
+void launch_window_blk(const WindowParams& p, int64_t rows, hipStream_t stream) {
   const int G = p.Hq / p.Hkv;
   const size_t lds = 3 * sizeof(int) * (static_cast<size_t>(p.B) + 1);
   const int64_t blocks = (rows + 16 * RT - 1) / (16 * RT) + p.B;  // (a bound)
-  const void* kern = reinterpret_cast<const void*>(&window_kernel<RT, kMode>);
+  const void* kern = reinterpret_cast<const void*>(&window_kernel<RT, kMode, kBlk>);
   const int64_t tasks = blocks * p.Hkv * ceil_div(G, kTiles / RT);
-  hipLaunchKernelGGL((window_kernel<RT, kMode>), dim3(grid_for(4 * tasks, kern, lds)), dim3(256), lds, stream, p);
+  hipLaunchKernelGGL((window_kernel<RT, kMode, kBlk>), dim3(grid_for(4 * tasks, kern, lds)), dim3(256), lds, stream, p);
+}
+
+// Blocks of 64 keys, but of 32 for windows of 16-row tasks over a K/V set the
+// caches do not hold: a window of 256 keys then ends within 32 keys of what
+// its task loads instead of 64, and the loads past it go to HBM (8 heads per
+// group, window 256: 64 x 8192 rows, 1.07 GB of K/V, 4585 us with 64-key
+// blocks, 4465 with 32; 8 x 8192 rows, 168 MB, 551 and 559).
+constexpr int64_t kFarBytes = 256ll << 20;  // the memory-side cache
+
+template <int RT, int kMode>
+void launch_window_rt(const WindowParams& p, int64_t rows, hipStream_t stream) {
+  if constexpr (kMode == kRectify) {
+    launch_window_blk<RT, kMode, 32>(p, rows, stream);
+  } else if constexpr (RT == 1) {
+    if (p.window_left >= 0 && p.kv_len_total * p.Hkv * (4 * kHeadDim) > kFarBytes)
+      launch_window_blk<RT, kMode, 32>(p, rows, stream);
+    else
+      launch_window_blk<RT, kMode, 64>(p, rows, stream);
+  } else {
+    launch_window_blk<RT, kMode, 64>(p, rows, stream);
+  }
 }
 
 // Launches the window kernel over at most `rows` query rows.

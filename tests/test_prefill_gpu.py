@@ -630,3 +630,23 @@ def test_window_attention_split_keeps_bounds_and_masks(rect_ext):
     torch.cuda.synchronize()
     uo, ul = _unsplit(d, -1, case.sm_scale, qo=qo, kv=kv)
     assert torch.equal(out.view(torch.int16), uo.view(torch.int16)) and torch.equal(lse, ul)
+
+
+@pytest.mark.parametrize("window_left", [0, 40, 255])
+def test_window_attention_over_a_far_pool(rect_ext, window_left):
+    """Windows of GQA-8 groups over a K/V set larger than the caches take
+    32-key blocks that skip key groups past a window's end: the same rows
+    against the oracle, with the entries named as part of a larger index."""
+    case = syn.prefill_case(qo_lens=[1, 17, 300, 64], kv_lens=[1, 40, 700, 64], hq=16, hkv=2, seed=81)
+    d = _dev_case(case)
+    idx = torch.zeros((1 << 28) // 1024 + 1, dtype=torch.int32, device="cuda")  # more than 256 MiB of K/V rows
+    idx[:d["idx"].numel()] = d["idx"]
+    out, lse = rect_ext.window_attention_return_lse(d["q"], d["k"], d["v"], d["qo"], d["kv"], idx, window_left,
+                                                    case.sm_scale)
+    torch.cuda.synchronize()
+    eo, el = orc.window_attention(_bf(case.q), _bf(case.k), _bf(case.v), case.qo_indptr, case.kv_indptr,
+                                  case.kv_indices, window_left=window_left, sm_scale=case.sm_scale)
+    got = bits(_host_bits(out))
+    for r in range(got.shape[0]):
+        assert rel_l2(got[r], bits(eo[r])) < 1e-2, r
+    np.testing.assert_allclose(lse.cpu().numpy(), el, atol=2e-4, rtol=1e-5)
