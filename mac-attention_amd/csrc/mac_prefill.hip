@@ -179,10 +179,11 @@ struct WindowParams {
   // plain window attention
   uint16_t* out;
   float* out_lse;
-  // split form: partial states of the pieces, and the most pieces they hold
+  // split form: partial states of the pieces, the most pieces they hold and
+  // the most row blocks that window_combine_kernel's grid covers
   float* part_o;
   float* part_ml;
-  int max_pieces;
+  int max_pieces, max_blocks;
   // fused rectification
   const uint16_t* src_q;
   const uint16_t* o_full;
@@ -255,9 +256,9 @@ __device__ __forceinline__ int scan256(int v, int* s_tmp, int& total) {
 // and follows from the batch: with W = sum of blocks x keys and NB blocks,
 // chunk = W / (max_pieces - NB) rounded up to whole 64-key blocks gives at
 // most W / chunk + NB <= max_pieces pieces.  Requests whose query ranges
-// overlap can hold more row blocks than the caller's row count allows for:
-// with no room for them the chunk is kNoChunk, every piece is a whole block
-// and writes its result itself.
+// overlap can hold more row blocks than the caller's row count allows for
+// (p.max_blocks), which is all the combining launch covers: the chunk is then
+// kNoChunk, every piece is a whole block and writes its result itself.
 constexpr int kNoChunk = 1 << 30;  // (a request has fewer keys)
 constexpr int kMinSplitKeys = 256;  // smallest chunk: a piece's prologue and state cost about as much
 
@@ -286,7 +287,7 @@ __device__ __forceinline__ int plan_pieces(const WindowParams& p, int* s_boff, i
     w = 0;
 #pragma unroll
     for (int i = 0; i < kWaves; ++i) w += s_w[i];
-    const int room = p.max_pieces - total_nb;
+    const int room = total_nb <= p.max_blocks ? p.max_pieces - total_nb : 0;
     const long long c = room > 0 ? ((w + room - 1) / room + 63) / 64 * 64 : kNoChunk;
     chunk = static_cast<int>(min(max(c, static_cast<long long>(kMinSplitKeys)), static_cast<long long>(kNoChunk)));
   }
@@ -1253,6 +1254,7 @@ extern "C" int mac_prefill_window_attention_ws_bf16(const MacWindowAttentionArgs
     p.part_o = static_cast<float*>(workspace);
     p.part_ml = reinterpret_cast<float*>(static_cast<char*>(workspace) + sp.o_bytes);
     p.max_pieces = sp.pieces;
+    p.max_blocks = static_cast<int>(sp.blocks);
     switch (row_tiles(p.Hq / p.Hkv)) {
       case 1: launch_split<1>(p, sp, s); break;
       case 2: launch_split<2>(p, sp, s); break;

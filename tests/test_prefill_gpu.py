@@ -632,6 +632,44 @@ def test_window_attention_split_keeps_bounds_and_masks(rect_ext):
     assert torch.equal(out.view(torch.int16), uo.view(torch.int16)) and torch.equal(lse, ul)
 
 
+def _row_block_bound(rows, batch, group):
+    """Row blocks a batch of disjoint query ranges can hold (the split's plan)."""
+    block = 16 * (1 if group > 4 else 2 if group > 2 else 4 if group > 1 else 8)
+    return min(rows, -(-rows // block) + batch)
+
+
+@pytest.mark.parametrize("hq,hkv,last,repeats", [
+    (32, 4, 640, 3),   # 16-row blocks
+    (16, 2, 320, 3),
+    (8, 2, 320, 5),    # 32-row blocks
+    (4, 2, 330, 7),    # 64-row blocks
+    (2, 2, 400, 9),    # 128-row blocks
+    (2, 2, 400, 2),    # one row block more than the count allows for
+])
+def test_window_attention_split_with_overlapping_queries(rect_ext, hq, hkv, last, repeats):
+    """Overlapping query ranges hold more row blocks than the row count allows
+    for but fewer than the workspace has pieces: every row is written, also
+    those that only the last request owns, with the unsplit call's bits."""
+    shared = last - 20  # rows [shared, last) belong to the last request alone
+    group = hq // hkv
+    case = syn.prefill_case(qo_lens=[last], kv_lens=[20000], hq=hq, hkv=hkv, seed=63)
+    d = _dev_case(case)
+    qo, kv = _i32(np.array([0, shared] * repeats + [0, last], np.int32)), _i32(np.array([0, 20000] * (repeats + 1), np.int32))
+    block = 16 * (1 if group > 4 else 2 if group > 2 else 4 if group > 1 else 8)
+    blocks = repeats * -(-shared // block) + -(-last // block)
+    bound = _row_block_bound(last, qo.shape[0] - 1, group)
+    print(f"overlap: G={group} {blocks} row blocks, bound {bound}", flush=True)
+    assert _workspace_bytes(d, qo=qo) > 0 and blocks > bound
+    out = torch.zeros_like(d["q"])
+    lse = torch.full(d["q"].shape[:2], 7.0, device="cuda")
+    rect_ext.window_attention_return_lse(d["q"], d["k"], d["v"], qo, kv, d["idx"], -1, case.sm_scale, out=out, out_lse=lse)
+    torch.cuda.synchronize()
+    uo, ul = _unsplit(d, -1, case.sm_scale, qo=qo, kv=kv)
+    own = slice(shared, last)  # (the shared rows are written by requests of two lengths, in no order)
+    assert torch.equal(out[own].view(torch.int16), uo[own].view(torch.int16)) and torch.equal(lse[own], ul[own])
+    assert not (lse == 7.0).any()
+
+
 @pytest.mark.parametrize("window_left", [0, 40, 255])
 def test_window_attention_over_a_far_pool(rect_ext, window_left):
     """Windows of GQA-8 groups over a K/V set larger than the caches take
