@@ -5,7 +5,7 @@
 // allocation):
 //
 //  1. match_decide  (one workgroup per (request, KV head) group, four or
-//     eight waves; for rings of more than 128 slots, a range-split probe scan
+//     eight waves; for rings of more than 192 slots, a range-split scan
 //     over (group, range) workgroups, then the decision kernel)
 //     Scans the request's ring of cached pre-RoPE queries for every query head
 //     of the group (squared L2, best = smallest distance, ties to the smaller
@@ -50,7 +50,9 @@
 //     complete_task_go[2 NG + 2 .. + 4]: the previous step's short groups,
 //     long groups and tokens / 64 (step_fuse_rule);
 //     complete_task_tile[NG]: span_attention's task counter (NG = N Hkv);
-//   match_dist/pos/slot[..., 0]: best (distance, position, slot) of the scan;
+//   match_dist/pos/slot[..., 0]: best (distance, position, slot) of the scan
+//     (of a probed ring, the slots whose probe passed); the other tiles: the
+//     ranges' bests, where the ring is scanned in ranges;
 //   partial_o / partial_lse: one (o, lse) partial per task and head;
 //   task_counts: [0] tasks, [1] tail tasks, [3] non-hit groups whose band spans
 //     more than one tile_tokens tile, [4] chunk C, [5] non-hit groups, [6]
@@ -751,11 +753,12 @@ __device__ __forceinline__ uint32_t pack_bf16x2(float a, float b) {
 // Larger rings are scanned by a separate launch over (group, slot range)
 // (kMode 1, `splits` ranges, scan_splits) that writes each
 // range's best into tile `range` of match_dist/pos/slot; match_decide then
-// reduces the tiles (kMode 2) instead of scanning.  kMode 0 scans and decides
+// reduces the tiles into tile 0 (kMode 2) instead of scanning.  kMode 0 scans and decides
 // in one workgroup per group.
 constexpr int kSplitSlots = 256;
 constexpr int kMinSplitSlots = 32;
-constexpr int kWholeRing = 128;
+constexpr int kProbeRanges = 3;
+constexpr int kWholeRing = 192;
 // complete_task_go / _tile entries beyond 2 N Hkv: the long-group flag, one
 // spare, the previous step's counts for the short-group rule, one spare
 constexpr int kTaskExtra = 6;
@@ -806,7 +809,7 @@ __device__ __forceinline__ void decide_group(const DecideParams& p, const float 
     }
     return;
   }
-  if (kMode == 0 && head_lane) {
+  if (head_lane) {  // (kMode 2: every lane read its ranges' tiles before the barrier ahead of this)
     p.match_dist[mo] = bd;
     p.match_pos[mo] = bp;
     p.match_slot[mo] = bs;
@@ -2346,20 +2349,32 @@ int fuse_tokens() {
   return x < 0 ? 0 : x;
 }
 
+// Rings of at least kProbeRanges ranges of kSplitSlots slots (and as many match
+// tiles) are probed.  A smaller ring is read in full: its best (distance,
+// position, slot) is reported for every head, also one without a hit, whose
+// best slots a probe would have pruned.
+bool probed_ring(int M, int max_match_tiles) {
+  return std::min(max_match_tiles, ceil_div(M, kSplitSlots)) >= kProbeRanges;
+}
+
 // Slot ranges of the ring scan (1: match_decide scans the ring itself).
-// Rings of at most kWholeRing slots take the deciding workgroup one or two
-// rounds of loads; larger ones are scanned by a launch of their own, whose
-// probe reads half of most rows, in ranges of up to kSplitSlots slots, fewer
-// where the groups alone would leave CUs idle: two workgroups per CU, down to
-// kMinSplitSlots slots (one round of loads), as far as there are match tiles.
-// Step times (us) scanned in one workgroup / split, 4K contexts, hit 0.5, GQA-8:
-// 1 request, ring 128: 41.3 / 40.8, 192: 45.2 / 41.1, 512: 61.9 / 41.3; 16
-// requests, ring 512: 72 / 56; 64, ring 512: 123 / 113.  256-slot ranges alone
-// (rings of 513 slots on): 1 request, ring 2048: 57.6 / 42.5.
+// Rings of at most kWholeRing slots take the deciding workgroup a few rounds
+// of loads; larger ones are scanned by a launch of their own, where the groups
+// alone would leave CUs idle: two workgroups per CU, down to kMinSplitSlots
+// slots (one round of loads), as far as there are match tiles.  A ring read in
+// full is split where that gives every group four or more ranges; a probed one
+// always, in ranges of at most kSplitSlots slots, since the probe reads half
+// of most rows.  Step times (us) scanned in one workgroup / split, GQA-4, 8 KV
+// heads, 2K contexts, hit 0.9: 1 request, ring 192: 35.8 / 35.9, 256: 37.9 /
+// 35.6, 512: 46.1 / 35.8; 16 requests, 192: 38.9 / 40.9, 512: 49.8 / 45.7; 24
+// requests (three ranges), 512: 55.7 / 61.1; 32, 512: 64.3 / 70.7.  256-slot
+// ranges alone for a probed ring of 2048 slots, 1 request: 57.6 / 42.5.
 int scan_splits(int M, int groups, int max_match_tiles, int cus) {
   if (M <= kWholeRing) return 1;
+  const bool probed = probed_ring(M, max_match_tiles);
+  if (!probed && 2 * groups > cus) return 1;
   const int most = std::min(max_match_tiles, ceil_div(M, kMinSplitSlots));
-  return std::max(1, std::min(most, std::max(ceil_div(M, kSplitSlots), ceil_div(2 * cus, groups))));
+  return std::max(1, std::min(most, std::max(probed ? ceil_div(M, kSplitSlots) : 1, ceil_div(2 * cus, groups))));
 }
 
 template <int G>
@@ -2570,8 +2585,8 @@ int mac::decode_impl(const MacDecodeArgs* a, void* stream_ptr, hipEvent_t* ev) {
   dp.task_counter = a->complete_task_tile + static_cast<int64_t>(N) * Hkv;
   // rings of more than kWholeRing slots are scanned by a separate (group,
   // range) launch, one match tile per range
-  dp.probe = match_probe();
   dp.splits = scan_splits(M, N * Hkv, a->max_match_tiles, cus);
+  dp.probe = match_probe() && probed_ring(M, a->max_match_tiles);
   dp.S = a->semantic_pos_ahead;
   dp.F = a->front_sink_tokens > 0 ? a->front_sink_tokens : 0;
   dp.gen_min_limit = a->gen_min_limit;

@@ -478,11 +478,13 @@ def test_small_step_chunks(partial, hkv, kv_lens, fuse, ext, monkeypatch):
 
 
 @pytest.mark.parametrize("ring,kv_lens,hkv", [
-    (128, [400, 90], 2),                 # the largest ring one workgroup scans
-    (129, [700, 100, 129, 130], 8),      # the smallest split one: five ranges, the last of one slot; unfilled rings
+    (128, [400, 90], 2),                 # scanned by the deciding workgroup
+    (192, [700, 100, 129, 130], 8),      # the largest ring that always is
+    (193, [700, 100, 193, 194], 8),      # the smallest split one: seven ranges of 28 slots, the last of 25; unfilled rings
     (300, [301, 5000], 4),               # a ring just full, and a wrapped one
     (512, [2300, 511, 513], 1),
-    (4500, [6000, 4499], 2),             # more ranges than a row of lanes reads in one pass
+    (1261, [1300, 2000], 2),             # tiles of 36: 36 ranges of 36, the last of one slot
+    (4500, [6000, 4499], 2),             # tiles of 16: 128 ranges of 36, three of them empty
 ])
 @pytest.mark.parametrize("group", [1, 3, 4, 8])
 def test_split_ring_scan(ring, kv_lens, hkv, group, ext):
@@ -493,8 +495,52 @@ def test_split_ring_scan(ring, kv_lens, hkv, group, ext):
     c = syn.random_case(batch=len(kv_lens), hq=group * hkv, hkv=hkv, kv_lens=kv_lens, capacity=ring,
                         semantic_pos_ahead=32, front_sink_tokens=8, hit_rate=0.6, match_lag=min(ring, 120) - 1, seed=ring)
     res = oracle_run(c)
-    for tile_slots in (16, 256):
+    for tile_slots in (16, 36, 256):
         dev = syn.to_device(torch, c)
         out, out_lse, ws = syn.run_decode(torch, ext, dev, c, max_context=6144, tile_tokens=32, match_tile_slots=tile_slots)
         torch.cuda.synchronize()
         _check_against_oracle(c, dev, out, out_lse, ws, res, what=f"split scan {ring} {tile_slots}")
+
+
+@pytest.mark.parametrize("ring,kv_lens,hkv,tile_slots", [
+    (100, [90, 400], 2, 16),              # scanned by the deciding workgroup
+    (129, [700, 100, 129, 130], 8, 16),
+    (193, [700, 100, 193, 194], 8, 16),   # scanned in ranges
+    (300, [301, 5000], 4, 32),
+    (512, [2300, 511, 513], 1, 32),
+    (512, [700], 8, 128),                 # four match tiles for 16 ranges
+    (512, [700], 8, 512),                 # one match tile: not split
+    (512, [600] * 64, 4, 32),             # a group per CU: not split
+    (512, [600] * 32, 4, 32),             # ranges of 128 slots
+    (1000, [1500, 999], 2, 512),          # two match tiles: ranges read in full
+    (1024, [3000, 900], 4, 32),           # probed
+])
+@pytest.mark.parametrize("group", [1, 4, 8])
+def test_best_match_is_in_tile_zero(ring, kv_lens, hkv, tile_slots, group, ext):
+    """match_dist/pos/slot hold the ring's overall best in tile 0, however the
+    ring is scanned: for every head where it is read in full, for the heads
+    with a hit where it is probed."""
+    if len(kv_lens) >= 32 and group != 4:
+        pytest.skip("one group size is enough for the large batches")
+    print(f"best match: ring={ring} kv={len(kv_lens)} x {kv_lens[0]} hkv={hkv} G={group}", flush=True)
+    c = syn.random_case(batch=len(kv_lens), hq=group * hkv, hkv=hkv, kv_lens=kv_lens, capacity=ring,
+                        semantic_pos_ahead=32, hit_rate=0.5, noise=0.2, match_lag=min(ring, 120) - 1, seed=ring,
+                        entry_builder="random")
+    dev = syn.to_device(torch, c)
+    _, _, ws = syn.run_decode(torch, ext, dev, c, max_context=6144, tile_tokens=32, match_tile_slots=tile_slots)
+    torch.cuda.synchronize()
+    hit, dist, pos, slot = (_np(ws[i])[:len(kv_lens)] for i in (3, 0, 1, 2))
+    dist, pos, slot = dist[..., 0], pos[..., 0], slot[..., 0]
+    probed = min(ws[0].shape[2], -(-ring // 256)) >= 3
+    assert 0 < hit.sum() < hit.size
+    for n, kv in enumerate(kv_lens):
+        past = kv - 1
+        filled = min(past, ring)
+        d = ((c.query_cache[n, :filled].astype(np.float64) - c.q_pre[n].astype(np.float64)) ** 2).sum(-1)  # [slots, heads]
+        for h in range(group * hkv):
+            if probed and not hit[n, h]:
+                continue
+            best = d[:, h].min()
+            assert 0 <= slot[n, h] < filled and pos[n, h] == syn.ring_slot_to_pos(past, ring, int(slot[n, h])), (n, h)
+            # (a 128-term fp32 sum is within 128 * 2^-24 < 1e-5 of its value)
+            assert abs(dist[n, h] - best) <= 1e-5 * best and d[slot[n, h], h] <= best * (1 + 2e-5), (n, h)
