@@ -961,7 +961,7 @@ __global__ void __launch_bounds__(256) window_combine_kernel(WindowParams p) {
   const int h = kHeads * (hc - hkv * nchunks) + tile / RT;  // head in the group
   const int r0 = 16 * (tile % RT);
   if (h >= G || r0 + col >= nrows) return;  // (window_kernel stored the lanes of whole rows only)
-  const int n = ceil_div(pos_last + 1, chunk);  // pieces with keys of these rows
+  const int n = __builtin_amdgcn_readfirstlane(ceil_div(pos_last + 1, chunk));  // pieces with keys of these rows
   auto slot = [&](int ch) {  // tile slot of chunk ch (window_kernel's task order)
     return (static_cast<int64_t>(s_boff[b] + ch * nb + blk) * per_piece + hc) * kTiles + tile;
   };
@@ -989,10 +989,13 @@ __global__ void __launch_bounds__(256) window_combine_kernel(WindowParams p) {
     o[1] *= keep;
 #pragma unroll
     for (int u = 0; u < kBatch; ++u) {
-      const float f = c0 + u < n ? fast_exp2(w[u] - mx) : 0.0f;
+      // (past the last piece: nothing, not its copy with weight 0, which may hold infinities)
+      const bool in = c0 + u < n;
+      const float f = in ? fast_exp2(w[u] - mx) : 0.0f;
+      const f32x4_t zero = {0.0f, 0.0f, 0.0f, 0.0f};
       lt += f * l[u];
-      o[0] += f * a[u][0];
-      o[1] += f * a[u][1];
+      o[0] += f * (in ? a[u][0] : zero);
+      o[1] += f * (in ? a[u][1] : zero);
     }
   }
   const float inv = lt > 0.0f ? 1.0f / lt : 0.0f;

@@ -670,6 +670,25 @@ def test_window_attention_split_with_overlapping_queries(rect_ext, hq, hkv, last
     assert not (lse == 7.0).any()
 
 
+def test_window_attention_split_keeps_infinities(rect_ext):
+    """A row's infinite value stays infinite, in whichever of its pieces the
+    key falls, and touches no other dim: the combining kernel adds no piece
+    with weight 0 (0 * inf is NaN)."""
+    case = syn.prefill_case(qo_lens=[1], kv_lens=[2500], hq=8, hkv=2, seed=71)  # 10 pieces of 256 keys, the last of 196
+    d = _dev_case(case)
+    assert _workspace_bytes(d) > 0
+    for key, dim, value in ((2499, 3, math.inf), (40, 64, -math.inf), (1300, 127, math.inf)):
+        d["v"][d["idx"][key].long(), 1, dim] = value
+    out, _ = rect_ext.window_attention_return_lse(d["q"], d["k"], d["v"], d["qo"], d["kv"], d["idx"], -1, case.sm_scale)
+    torch.cuda.synchronize()
+    out = out.float()[0]
+    assert torch.isfinite(out[:4]).all()
+    assert (out[4:, [3, 127]] == math.inf).all() and (out[4:, 64] == -math.inf).all()
+    finite = torch.ones(128, dtype=torch.bool)
+    finite[[3, 64, 127]] = False
+    assert torch.isfinite(out[4:][:, finite.to(out.device)]).all()
+
+
 @pytest.mark.parametrize("window_left", [0, 40, 255])
 def test_window_attention_over_a_far_pool(rect_ext, window_left):
     """Windows of GQA-8 groups over a K/V set larger than the caches take
