@@ -22,8 +22,8 @@
 // v_mfma_f32_16x16x32_bf16 as the decode kernel does, with 16 query rows in
 // place of the GQA heads: the lane holding row l%16 keeps that row's softmax
 // state and 32 O^T accumulators per head.  A workgroup takes rows of one
-// request and query heads of one KV head, 128 (row, head) columns in all; its
-// four waves share double-buffered LDS K/V tiles.  The layouts are described
+// request and query heads of one KV head, 128 or 64 (row, head) columns in all;
+// its four waves share double-buffered LDS K/V tiles.  The layouts are described
 // above window_kernel.
 
 #include <hip/hip_runtime.h>
@@ -167,7 +167,7 @@ __global__ void __launch_bounds__(256) downdate_kernel(const uint16_t* __restric
 // ------------------------------------------------------ window attention ----
 
 constexpr int kMaxB = 4096;  // requests handled by the in-workgroup planner
-constexpr int kTiles = 8;    // column tiles (16 query rows of one head) of a task
+constexpr int kTiles = 8;    // column tiles (16 query rows of one head) of a wide task
 
 struct WindowParams {
   const uint16_t* q;  // attention queries [total_q, Hq, 128]
@@ -329,15 +329,17 @@ __device__ __forceinline__ int request_of(const int* s_boff, int B, int piece) {
 // fed to the PV product as bf16 hi + lo, and the downdate and ring write as
 // epilogue).
 //
-// A task is 8 column tiles of one KV head: a tile is 16 consecutive query
-// rows of one query head, and the 8 are RT row tiles x 8 / RT heads, RT
-// picked from the GQA group so that no tile is wasted on an absent head (G >
-// 4: 16 rows x 8 heads; 3, 4: 32 x 4; 2: 64 x 2; 1: 128 x 1).  Each of the
-// four waves owns two of them, so every K and V operand a wave reads from LDS
-// feeds 32 columns whatever the group size.  K/V rows are staged in
-// double-buffered LDS tiles of kBlk keys: 64 (one barrier and one round of
-// address work per 64 keys), or 32 (fused form, whose epilogue also holds the
-// full state's rows in LDS, and far windows, see launch_window_rt).  Per wave and 32 keys:
+// A task is 4 kPer column tiles of one KV head: a tile is 16 consecutive query
+// rows of one query head, each of the four waves owns kPer of them.  Wide tasks
+// (kPer 2) are RT row tiles x 8 / RT heads, RT picked from the GQA group so
+// that no tile is wasted on an absent head (G > 4: 16 rows x 8 heads; 3, 4: 32
+// x 4; 2: 64 x 2; 1: 128 x 1), so that every K and V operand a wave reads from
+// LDS feeds 32 columns whatever the group size.  Narrow tasks (kPer 1, RT 1: 16
+// rows x 4 heads) have the shorter chain (see narrow_tasks).  K/V rows are
+// staged in double-buffered LDS tiles of kBlk keys: 64 (one barrier and one
+// round of address work per 64 keys), or 32 (fused form, whose epilogue also
+// holds the full state's rows in LDS, narrow tasks, and see long_blocks).  Per
+// wave and 32 keys:
 //  * S^T = K Q^T: the A operand of score tile t, row m, is key 16 t + m; the
 //    lane holding column col ends up with the scores of keys 16 t + 4 quad +
 //    (0..3), quad = lane / 16.
@@ -369,12 +371,13 @@ __device__ __forceinline__ int request_of(const int* s_boff, int B, int piece) {
 constexpr int kKRow = 16;  // 16-byte units per staged K row
 constexpr int kVRow = 18;  // per staged V row: 256 + 32
 
-template <int RT, int kMode, int kBlk>
-__global__ void __launch_bounds__(256, 2) window_kernel(WindowParams p) {
+template <int RT, int kPer, int kMode, int kBlk>
+__global__ void __launch_bounds__(256, (kPer == 1 && kMode == kPlain) ? 3 : 2) window_kernel(WindowParams p) {
   constexpr bool kFused = kMode == kRectify;
-  constexpr int kHeads = kTiles / RT;   // query heads of a task
+  constexpr int kTask = kWaves * kPer;  // column tiles of a task
+  constexpr int kHeads = kTask / RT;    // query heads of a task
   constexpr int kRowsT = 16 * RT;       // query rows of a task
-  constexpr bool kFarWindow = kMode == kPlain && kBlk == 32;  // (launch_window_rt)
+  constexpr bool kTrim = kMode == kPlain && kBlk == 32;  // no loads of 16-key groups past the keys' end
   constexpr int kSub = kBlk / 32;
   constexpr int kLd = kBlk / 16;  // keys each thread stages a chunk of
   // dynamic: s_boff[B + 1] piece offsets, s_qo[B + 1] / s_kv[B + 1] the
@@ -386,7 +389,7 @@ __global__ void __launch_bounds__(256, 2) window_kernel(WindowParams p) {
   __shared__ int s_part[kWaves];
   __shared__ uint4 s_k[2][kBlk * kKRow];
   __shared__ uint4 s_v[2][kBlk * kVRow];
-  __shared__ uint32_t s_bad[2][kWaves][2];  // per wave: its keys (of each 32) that have no pool row
+  __shared__ __align__(16) uint32_t s_bad[2][kWaves * kSub];  // per wave: its keys (of each 32) that have no pool row
 
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -405,7 +408,7 @@ __global__ void __launch_bounds__(256, 2) window_kernel(WindowParams p) {
   // head takes 16 16-byte units from unit 16 e + (e >> 2) on (the extra unit
   // per four pairs spreads the rows over the banks; a wave's direct copy
   // fills four pairs, one contiguous 1 KiB run)
-  __shared__ uint4 s_of[kFused ? 128 * 16 + 32 : 1];
+  __shared__ uint4 s_of[kFused ? kTask * (16 * 16 + 4) : 1];
   const int nchunks = ceil_div(G, kHeads);
   const int per_piece = Hkv * nchunks;
   const int total_tasks = s_boff[B] * per_piece;
@@ -425,9 +428,13 @@ __global__ void __launch_bounds__(256, 2) window_kernel(WindowParams p) {
   for (int s = 0; s < 4; ++s) rd_k[s] = &s_k[0][0] + col * kKRow + ((4 * s + quad) ^ col);
   const uint16_t* const rd_v =
       reinterpret_cast<const uint16_t*>(&s_v[0][0]) + (4 * quad + (col >> 2)) * (kVRow * 8) + 4 * (col & 3);
-  // the wave's tiles c = 0, 1: task head and first row in the task
-  const int th0 = (2 * wave) / RT, th1 = (2 * wave + 1) / RT;
-  const int tr0 = 16 * ((2 * wave) % RT), tr1 = 16 * ((2 * wave + 1) % RT);
+  // the wave's tiles c < kPer: task head and first row in the task
+  int th[kPer], tr[kPer];
+#pragma unroll
+  for (int c = 0; c < kPer; ++c) {
+    th[c] = (kPer * wave + c) / RT;
+    tr[c] = 16 * ((kPer * wave + c) % RT);
+  }
 
   // Task order, by form (measured at 64 requests x 8192 rows, S = 256):
   //  * windowed (plain, window_left >= 0): (KV head, head chunk) major, row
@@ -481,18 +488,19 @@ __global__ void __launch_bounds__(256, 2) window_kernel(WindowParams p) {
     const int pos_last = pos0 + nrows - 1;
     if (kMode == kSplit && key_lo > pos_last) continue;  // (past every row: the combine skips it too)
     // tile c of the wave: lane's row in the task, position, first key of its window
-    const bool live0 = hg0 + th0 < G && tr0 < nrows, live1 = hg0 + th1 < G && tr1 < nrows;
-    const bool live = live0 || live1;
-    int row[2], wlo[2];
-    bool row_ok[2];
+    bool live = false;
+    int row[kPer], wlo[kPer];
+    bool row_ok[kPer];
 #pragma unroll
-    for (int c = 0; c < 2; ++c) {
-      row[c] = (c == 0 ? tr0 : tr1) + col;
-      row_ok[c] = row[c] < nrows && (c == 0 ? live0 : live1);
+    for (int c = 0; c < kPer; ++c) {
+      const bool live_c = hg0 + th[c] < G && tr[c] < nrows;
+      live = live || live_c;
+      row[c] = tr[c] + col;
+      row_ok[c] = row[c] < nrows && live_c;
       wlo[c] = wl < 0 ? 0 : max(pos0 + row[c] - wl, 0);
     }
     // first and last row of the wave's tiles (uniform), for the mask-free test
-    const int rf = min(tr0, tr1), rl = min(max(tr0, tr1) + 15, nrows - 1);
+    const int rf = min(tr[0], tr[kPer - 1]), rl = min(max(tr[0], tr[kPer - 1]) + 15, nrows - 1);
     const int wlo_f = wl < 0 ? 0 : max(pos0 + rf - wl, 0), wlo_l = wl < 0 ? 0 : max(pos0 + rl - wl, 0);
     // this request's kv_indices; entry offsets fit 32 bits (fewer than 2^30
     // entries, checked on the host), so a load is a uniform base plus a
@@ -517,20 +525,22 @@ __global__ void __launch_bounds__(256, 2) window_kernel(WindowParams p) {
     // fused form: the epilogue's inputs that do not depend on the attention,
     // loaded now so that their latency hides behind it
     auto grow = [&](int r) { return static_cast<int64_t>(s_qo[b]) + r_local + (r < nrows ? r : 0); };
-    const int64_t grow0 = grow(row[0]), grow1 = grow(row[1]);
+    int64_t grow_c[kPer];
+#pragma unroll
+    for (int c = 0; c < kPer; ++c) grow_c[c] = grow(row[c]);
     int req = 0, before = 0;
-    float lse_full[2] = {0.0f, 0.0f};
+    float lse_full[kPer] = {};
     if (kFused) {
       req = p.req_ids[b];
       const bool req_ok = req >= 0 && req < p.R;
       before = p.rl_by_batch ? p.request_length[b] : p.request_length[req_ok ? req : 0];
-      lse_full[0] = p.lse_full[grow0 * Hq + hkv * G + min(hg0 + th0, G - 1)];
-      lse_full[1] = p.lse_full[grow1 * Hq + hkv * G + min(hg0 + th1, G - 1)];
+#pragma unroll
+      for (int c = 0; c < kPer; ++c) lse_full[c] = p.lse_full[grow_c[c] * Hq + hkv * G + min(hg0 + th[c], G - 1)];
     }
     // Fused form: the task's pre-RoPE query rows (copied into the ring with
     // the q_post NaN marker) and the full state's o rows (into s_of for the
-    // epilogue) -- 128 (row, head) pairs x 16 parts of 16 bytes, 8 rounds of
-    // one part per thread -- move with the K/V stream, so that this traffic
+    // epilogue) -- 16 kTask (row, head) pairs x 16 parts of 16 bytes, kTask
+    // rounds of one part per thread -- move with the K/V stream, so that this traffic
     // overlaps the compute-bound key blocks instead of adding an HBM-bound
     // load round after them (every workgroup runs its task in step with the
     // others).  A round's loads go out behind a block's K/V loads; its query
@@ -538,7 +548,7 @@ __global__ void __launch_bounds__(256, 2) window_kernel(WindowParams p) {
     // straight into LDS (global_load_lds_dwordx4: no registers; waited for at
     // the next block's staging and barrier).  Round k, thread t: pair 16 k +
     // t / 16, part t % 16.
-    constexpr int kCq = 8;
+    constexpr int kCq = kTask;
     const int cq_part = tid & 15;
     const bool cq_req = kFused && req >= 0 && req < p.R;
     int cq = 0;               // rounds issued (uniform)
@@ -572,11 +582,11 @@ __global__ void __launch_bounds__(256, 2) window_kernel(WindowParams p) {
     // zeroed): such a lane's results are never stored, and each column keeps
     // its own softmax state.  With no select on the loaded values no wait
     // follows the loads: the Q rows and the first entries are one round.
-    uint4 qreg[2][4];
+    uint4 qreg[kPer][4];
 #pragma unroll
-    for (int c = 0; c < 2; ++c) {
-      const int h = hkv * G + min(hg0 + (c == 0 ? th0 : th1), G - 1);
-      const uint16_t* qp = p.q + ((c == 0 ? grow0 : grow1) * Hq + h) * kHeadDim;
+    for (int c = 0; c < kPer; ++c) {
+      const int h = hkv * G + min(hg0 + th[c], G - 1);
+      const uint16_t* qp = p.q + (grow_c[c] * Hq + h) * kHeadDim;
 #pragma unroll
       for (int s = 0; s < 4; ++s) qreg[c][s] = *reinterpret_cast<const uint4*>(qp + 8 * (4 * s + quad));
     }
@@ -588,10 +598,12 @@ __global__ void __launch_bounds__(256, 2) window_kernel(WindowParams p) {
     // VALU; the plain form cannot do that, since its P is bf16 hi alone and
     // the sum of that is ~2^-9 off per key, beyond what its lse output allows.
     // vt[c]: the scaled score past which m[c] moves (-inf: none seen yet).
-    float m[2] = {kNegBig, kNegBig}, vt[2] = {-INFINITY, -INFINITY};
-    f32x4_t acc[2][8], l[2];
+    float m[kPer], vt[kPer];
+    f32x4_t acc[kPer][8], l[kPer];
 #pragma unroll
-    for (int c = 0; c < 2; ++c) {
+    for (int c = 0; c < kPer; ++c) {
+      m[c] = kNegBig;
+      vt[c] = -INFINITY;
       l[c] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
       for (int dt = 0; dt < 8; ++dt) acc[c][dt] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
@@ -608,7 +620,7 @@ __global__ void __launch_bounds__(256, 2) window_kernel(WindowParams p) {
       ok = 0;
 #pragma unroll
       for (int i = 0; i < kLd; ++i) {
-        if (kFarWindow && base + 16 * i >= end) continue;  // (uniform: none of these 16 keys exists)
+        if (kTrim && base + 16 * i >= end) continue;  // (uniform: none of these 16 keys exists)
         const bool in = base + ld_key + 16 * i < end && static_cast<unsigned>(raw[i]) < pool_rows;
         ok |= in ? 1u << i : 0u;
         const char* at = kbase + static_cast<uint64_t>(static_cast<uint32_t>(in ? raw[i] : 0)) * row_bytes;
@@ -677,8 +689,8 @@ __global__ void __launch_bounds__(256, 2) window_kernel(WindowParams p) {
             }
           }
           if (lane == 0) {
-            s_bad[buf][wave][0] = bad[0];
-            s_bad[buf][wave][1] = bad[1];
+#pragma unroll
+            for (int h = 0; h < kSub; ++h) s_bad[buf][wave * kSub + h] = bad[h];
           }
         }
         __syncthreads();  // the block is visible; every wave is done with the block before last (same buffer)
@@ -704,7 +716,7 @@ __global__ void __launch_bounds__(256, 2) window_kernel(WindowParams p) {
           const uint16_t* vtile = rd_v + (buf * (kBlk * kVRow) + sub * (32 * kVRow)) * 8;
           uint32_t bad = 0;
 #pragma unroll
-          for (int w = 0; w < kWaves; ++w) bad |= s_bad[buf][w][sub];
+          for (int w = 0; w < kWaves; ++w) bad |= s_bad[buf][w * kSub + sub];
           bad = __builtin_amdgcn_readfirstlane(bad);
           uint4 ka[2][4];
 #pragma unroll
@@ -718,9 +730,9 @@ __global__ void __launch_bounds__(256, 2) window_kernel(WindowParams p) {
                                              0, 1, 2, 3, 4, 5, 6, 7);
           // raw scores, the four accumulation chains interleaved (a tile
           // without rows is computed but never stored)
-          f32x4_t c4[2][2];
+          f32x4_t c4[kPer][2];
 #pragma unroll
-          for (int c = 0; c < 2; ++c)
+          for (int c = 0; c < kPer; ++c)
 #pragma unroll
             for (int t = 0; t < 2; ++t) c4[c][t] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
@@ -728,23 +740,24 @@ __global__ void __launch_bounds__(256, 2) window_kernel(WindowParams p) {
 #pragma unroll
             for (int t = 0; t < 2; ++t) {
 #pragma unroll
-              for (int c = 0; c < 2; ++c)
+              for (int c = 0; c < kPer; ++c)
                 c4[c][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(ka[t][s]), as_bf16x8(qreg[c][s]), c4[c][t], 0, 0, 0);
             }
           // keys inside every row's range, all present, need no masks
           if (kb < all_lo || kb + 32 > all_hi || bad != 0) {
 #pragma unroll
-            for (int c = 0; c < 2; ++c) {
-              const int pos = pos0 + row[c];
-              const int r_lo = seg == 0 ? 0 : wlo[c], r_hi = seg == 0 ? min(p.F, wlo[c]) : pos + 1;
+            for (int c = 0; c < kPer; ++c) {
+              // the row's keys [r_lo, r_hi) of the 32 as a bit mask: with two
+              // comparisons per key instead, a short window's two masked
+              // blocks cost a task 0.4 us
+              const int r_lo = seg == 0 ? 0 : wlo[c], r_hi = seg == 0 ? min(p.F, wlo[c]) : pos0 + row[c] + 1;
+              const int lo_k = min(max(r_lo - kb, 0), 32), hi_k = min(max(min(r_hi, seg_hi) - kb, 0), 32);
+              const uint64_t range = ((1ull << hi_k) - 1) & ~((1ull << lo_k) - 1);
+              const uint32_t keep = (static_cast<uint32_t>(range) & ~bad) >> (4 * quad);
 #pragma unroll
               for (int t = 0; t < 2; ++t)
 #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                  const int k = 16 * t + 4 * quad + r;
-                  const bool keep = kb + k >= r_lo && kb + k < min(r_hi, seg_hi) && ((bad >> k) & 1) == 0;
-                  c4[c][t][r] = keep ? c4[c][t][r] : -INFINITY;
-                }
+                for (int r = 0; r < 4; ++r) c4[c][t][r] = (keep >> (16 * t + r)) & 1 ? c4[c][t][r] : -INFINITY;
             }
           }
           // lazy move of the reference point: p <= 2^8 stays exact in fp32.
@@ -755,16 +768,18 @@ __global__ void __launch_bounds__(256, 2) window_kernel(WindowParams p) {
           // and l are still zero, and the rescale by 2^(kNegBig - m_new) = 0
           // leaves them zero).  The softmax scale is applied inside exp2:
           // m[c] is a raw score, p = 2^(q_scale (s - m)).
-          float bmax[2];
+          float bmax[kPer];
+          bool past = false;
 #pragma unroll
-          for (int c = 0; c < 2; ++c) {
+          for (int c = 0; c < kPer; ++c) {
             const float sv[8] = {c4[c][0][0], c4[c][0][1], c4[c][0][2], c4[c][0][3],
                                  c4[c][1][0], c4[c][1][1], c4[c][1][2], c4[c][1][3]};
             bmax[c] = max8_nonan(sv);
+            past = past || bmax[c] * p.q_scale > vt[c];
           }
-          if (__any(bmax[0] * p.q_scale > vt[0] || bmax[1] * p.q_scale > vt[1])) {
+          if (__any(past)) {
 #pragma unroll
-            for (int c = 0; c < 2; ++c) {
+            for (int c = 0; c < kPer; ++c) {
               const float bm = quad_max(bmax[c]);
               const float m_new = max3_nonan(m[c], bm, bm);
               const float alpha = fast_exp2((m[c] - m_new) * p.q_scale);
@@ -776,9 +791,9 @@ __global__ void __launch_bounds__(256, 2) window_kernel(WindowParams p) {
               for (int dt = 0; dt < 8; ++dt) acc[c][dt] *= alpha;
             }
           }
-          bf16x8_t pb[2], pl[2];
+          bf16x8_t pb[kPer], pl[kPer];
 #pragma unroll
-          for (int c = 0; c < 2; ++c) {
+          for (int c = 0; c < kPer; ++c) {
             const float mo = -m[c] * p.q_scale;
             float psum = 0.0f;
 #pragma unroll
@@ -799,7 +814,7 @@ __global__ void __launch_bounds__(256, 2) window_kernel(WindowParams p) {
           if (kFused) {
             const bf16x8_t ones = as_bf16x8(make_uint4(0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u));
 #pragma unroll
-            for (int c = 0; c < 2; ++c) {
+            for (int c = 0; c < kPer; ++c) {
               l[c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, pb[c], l[c], 0, 0, 0);
               l[c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, pl[c], l[c], 0, 0, 0);
             }
@@ -807,7 +822,7 @@ __global__ void __launch_bounds__(256, 2) window_kernel(WindowParams p) {
 #pragma unroll
           for (int dt = 0; dt < 8; ++dt)
 #pragma unroll
-            for (int c = 0; c < 2; ++c) {
+            for (int c = 0; c < kPer; ++c) {
               acc[c][dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(va[dt], pb[c], acc[c][dt], 0, 0, 0);
               if (kFused) acc[c][dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(va[dt], pl[c], acc[c][dt], 0, 0, 0);
             }
@@ -829,8 +844,8 @@ __global__ void __launch_bounds__(256, 2) window_kernel(WindowParams p) {
       // the piece's unnormalised state: O^T accumulators as the lanes hold
       // them, and per column its reference point (log2 units) and sum
 #pragma unroll
-      for (int c = 0; c < 2; ++c) {
-        const int64_t tile = static_cast<int64_t>(t) * kTiles + 2 * wave + c;
+      for (int c = 0; c < kPer; ++c) {
+        const int64_t tile = static_cast<int64_t>(t) * kTask + kPer * wave + c;
         const float lt = quad_sum(l[c][0]);
         f32x4_t* po = reinterpret_cast<f32x4_t*>(p.part_o) + tile * 8 * 64 + lane;
         if (!row_ok[c]) continue;
@@ -845,11 +860,11 @@ __global__ void __launch_bounds__(256, 2) window_kernel(WindowParams p) {
     }
     if (!kFused) {
 #pragma unroll
-      for (int c = 0; c < 2; ++c) {
+      for (int c = 0; c < kPer; ++c) {
         const float lt = quad_sum(l[c][0]);
         if (!row_ok[c]) continue;
         const float inv = lt > 0.0f ? 1.0f / lt : 0.0f;
-        const int64_t at = (c == 0 ? grow0 : grow1) * Hq + hkv * G + hg0 + (c == 0 ? th0 : th1);
+        const int64_t at = grow_c[c] * Hq + hkv * G + hg0 + th[c];
         uint16_t* op = p.out + at * kHeadDim + 4 * quad;
 #pragma unroll
         for (int dt = 0; dt < 8; ++dt) {
@@ -868,12 +883,11 @@ __global__ void __launch_bounds__(256, 2) window_kernel(WindowParams p) {
     if (before < 0) before = 0;
     const uint2* of2 = reinterpret_cast<const uint2*>(s_of);
 #pragma unroll
-    for (int c = 0; c < 2; ++c) {
+    for (int c = 0; c < kPer; ++c) {
       if (!row_ok[c]) continue;
       const int local = r_local + row[c];  // row index within the request
       const int slot = static_cast<int>((static_cast<int64_t>(before) + local) % p.M);
-      const int th = c == 0 ? th0 : th1;
-      const int64_t at = (static_cast<int64_t>(req) * p.M + slot) * Hq + hkv * G + hg0 + th;
+      const int64_t at = (static_cast<int64_t>(req) * p.M + slot) * Hq + hkv * G + hg0 + th[c];
       const bool empty = pos0 + row[c] + 1 - p.S <= (sink ? p.F : 0);  // nothing left after the downdate
       const float lt = l[c][0];
       const float inv = lt > 0.0f ? 1.0f / lt : 0.0f;
@@ -887,7 +901,7 @@ __global__ void __launch_bounds__(256, 2) window_kernel(WindowParams p) {
         d = downdate_control(lse_full[c], lse_w);
       }
       // the full state's o of the lane's row, dims 16 dt + 4 quad .. + 3, from s_of
-      const int e = row[c] * kHeads + th;
+      const int e = row[c] * kHeads + th[c];
       const uint2* of = of2 + 2 * (16 * e + (e >> 2)) + quad;
       uint16_t* ap = p.attn_cache + at * kHeadDim + 4 * quad;
 #pragma unroll
@@ -1054,6 +1068,13 @@ int device_cus() {
   return v;
 }
 
+// Tasks that `rows` query rows of B requests of about equal length make in
+// blocks of 16 rt rows and chunks of `heads` heads.
+int64_t expected_tasks(int64_t rows, int B, int Hq, int Hkv, int rt, int heads) {
+  const int64_t per_request = (rows + B - 1) / B;
+  return B * ((per_request + 16 * rt - 1) / (16 * rt)) * Hkv * ceil_div(Hq / Hkv, heads);
+}
+
 // Split over keys (causal attention over whole prefixes, window_left < 0):
 // pieces of the batch a split call plans for, or 0 where the row blocks alone
 // give the GPU enough work.  A task per (row block, head chunk) streams its
@@ -1100,52 +1121,104 @@ template <int RT>
 void launch_split(const WindowParams& p, const Split& sp, hipStream_t stream) {
   const int64_t per_piece = static_cast<int64_t>(p.Hkv) * ceil_div(p.Hq / p.Hkv, kTiles / RT);
   const size_t lds = sizeof(int) * (static_cast<size_t>(p.B) + 1);  // of one array over the requests
-  const void* kern = reinterpret_cast<const void*>(&window_kernel<RT, kSplit, 64>);
-  hipLaunchKernelGGL((window_kernel<RT, kSplit, 64>), dim3(grid_for(4 * sp.pieces * per_piece, kern, 3 * lds)), dim3(256),
+  const void* kern = reinterpret_cast<const void*>(&window_kernel<RT, 2, kSplit, 64>);
+  hipLaunchKernelGGL((window_kernel<RT, 2, kSplit, 64>), dim3(grid_for(4 * sp.pieces * per_piece, kern, 3 * lds)), dim3(256),
                      3 * lds, stream, p);
   hipLaunchKernelGGL((window_combine_kernel<RT>), dim3(static_cast<unsigned>(sp.blocks * per_piece * kTiles)), dim3(256),
                      2 * lds, stream, p);
 }
 
-template <int RT, int kMode, int kBlk>
-void launch_window_blk(const WindowParams& p, int64_t rows, hipStream_t stream) {
+template <int RT, int kPer, int kMode, int kBlk>
+void launch_window_as(const WindowParams& p, int64_t rows, hipStream_t stream) {
   const int G = p.Hq / p.Hkv;
   const size_t lds = 3 * sizeof(int) * (static_cast<size_t>(p.B) + 1);
   const int64_t blocks = (rows + 16 * RT - 1) / (16 * RT) + p.B;  // (a bound)
-  const void* kern = reinterpret_cast<const void*>(&window_kernel<RT, kMode, kBlk>);
-  const int64_t tasks = blocks * p.Hkv * ceil_div(G, kTiles / RT);
-  hipLaunchKernelGGL((window_kernel<RT, kMode, kBlk>), dim3(grid_for(4 * tasks, kern, lds)), dim3(256), lds, stream, p);
+  const void* kern = reinterpret_cast<const void*>(&window_kernel<RT, kPer, kMode, kBlk>);
+  const int64_t tasks = blocks * p.Hkv * ceil_div(G, kWaves * kPer / RT);
+  hipLaunchKernelGGL((window_kernel<RT, kPer, kMode, kBlk>), dim3(grid_for(4 * tasks, kern, lds)), dim3(256), lds, stream, p);
 }
 
-// Blocks of 64 keys, but of 32 for windows of 16-row tasks over a K/V set the
-// caches do not hold: a window of 256 keys then ends within 32 keys of what
-// its task loads instead of 64, and the loads past it go to HBM (8 heads per
-// group, window 256: 64 x 8192 rows, 1.07 GB of K/V, 4585 us with 64-key
-// blocks, 4465 with 32; 8 x 8192 rows, 168 MB, 551 and 559).
+// Narrow tasks (16 rows x 4 heads, one column tile per wave) or wide ones
+// (8 tiles, two per wave).  A narrow task's chain over its keys takes 25 us
+// per 1000 keys where a wide one's takes 31, and more of them run side by
+// side (three workgroups per CU); a wide task does twice the columns or more
+// with the same reads.  So narrow tasks serve the calls that leave the GPU
+// partly idle, where only the chain counts: as many narrow tasks as CUs, or
+// two per CU where wide tasks would fill at most half of them (a quarter with
+// a window: its wide chains are hardly longer).  And those whose requests
+// have too few rows for a wide task's rows, at any batch.  Times in us,
+// narrow / wide, 1000 keys or a window of 256, 4 heads per group but as said:
+//   64 rows 27 / 33; 64 rows of 8 heads 28 / 33, of 1 head 26 / 31;
+//   8 x 64 rows over 1500 keys (256 narrow) 40 / 49; 512 rows, window, 13 / 16;
+//   64 x 4 rows (512, as many wide) 29 / 36; 1100 x 16 rows, 300 keys, 184 / 258;
+//   16 x 64 rows (512, 256 wide) 38 / 36; window 19.8 / 19.2; 1 head 29 / 32
+//   (128 wide) and 16.6 / 14.4; 4 x 256 rows of 1 head, window (512, 64 wide),
+//   15.1 / 17.0; 64 x 64 rows 83 / 68.
+// Fused form (two workgroups per CU either way): 8 x 100 rows (448 narrow) 19.4 /
+// 22.6; 32 x 40 rows (768, 512 wide) 27.5 / 29.2, of 2 heads (256 wide) 25.9 /
+// 23.0; 32 x 100 rows (1792) 64.7 / 63.8.
+template <int kMode>
+bool narrow_tasks(const WindowParams& p, int64_t rows) {
+  const int64_t cus = device_cus();
+  const int rt = row_tiles(p.Hq / p.Hkv);
+  const int64_t narrow = expected_tasks(rows, p.B, p.Hq, p.Hkv, 1, kWaves);
+  const int64_t wide = expected_tasks(rows, p.B, p.Hq, p.Hkv, rt, kTiles / rt);
+  if (kMode == kRectify) return narrow <= 2 * cus || (narrow <= 3 * cus && 2 * narrow <= 3 * wide);
+  return 4 * narrow <= 5 * wide || narrow <= cus ||
+         (narrow <= 2 * cus && wide <= (p.window_left < 0 ? cus / 2 : cus / 4));
+}
+
+// Blocks of 32 or 64 keys for the wide tasks of 16-row blocks (plain form, 5
+// or more heads per group).  64 (half of the barriers) pay where several row
+// blocks share a request's keys: over whole prefixes, and with a window while
+// the GPU has more than a round of tasks; and for single blocks over whole
+// prefixes while it has at most one task per CU.  Elsewhere 32, whose window
+// ends nearer to what it loads and which waits for fewer keys at a time.  32
+// also for windows over a K/V set that the caches do not hold (the loads past a
+// window's end go to HBM) and for batches whose request offsets leave a CU no
+// room for two workgroups with 64.  Times in us, 64 / 32 (8 heads per group):
+// 30 x 100 rows over 1500 keys 125 / 129; 8 x 200 over 200, 17.7 / 18.9; 8 x
+// 8192, window 256, 553 / 558; 1 row over 3000 keys 81 / 86; 96 requests of 1
+// row over 1500 keys (384 tasks) 78 / 69; 500 x 16 rows over 300 keys 120 / 116;
+// 16 x 64 rows, window 256, 19.0 / 18.0; 1100 x 16 over 300 keys 287 / 231; 64
+// x 8192, window 256 (1.07 GB of K/V), 4640 / 4470.
 constexpr int64_t kFarBytes = 256ll << 20;  // the memory-side cache
 
+bool long_blocks(const WindowParams& p, int64_t rows, size_t request_bytes) {
+  const int64_t cus = device_cus();
+  const int64_t tasks = expected_tasks(rows, p.B, p.Hq, p.Hkv, 1, kTiles);
+  const int64_t far = std::min(p.kv_len_total, p.pool_tokens) * p.Hkv * (4 * kHeadDim);
+  if (p.window_left >= 0 && far > kFarBytes) return false;
+  int per_cu = 0;
+  const void* kern = reinterpret_cast<const void*>(&window_kernel<1, 2, kPlain, 64>);
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, 256, request_bytes) != hipSuccess || per_cu < 2) return false;
+  const bool shared = rows > 16 * static_cast<int64_t>(p.B);
+  return p.window_left < 0 ? shared || tasks <= cus : shared && tasks > 2 * cus;
+}
+
 template <int RT, int kMode>
-void launch_window_rt(const WindowParams& p, int64_t rows, hipStream_t stream) {
+void launch_window_wide(const WindowParams& p, int64_t rows, hipStream_t stream) {
   if constexpr (kMode == kRectify) {
-    launch_window_blk<RT, kMode, 32>(p, rows, stream);
+    launch_window_as<RT, 2, kMode, 32>(p, rows, stream);
   } else if constexpr (RT == 1) {
-    if (p.window_left >= 0 && p.kv_len_total * p.Hkv * (4 * kHeadDim) > kFarBytes)
-      launch_window_blk<RT, kMode, 32>(p, rows, stream);
+    if (long_blocks(p, rows, 3 * sizeof(int) * (static_cast<size_t>(p.B) + 1)))
+      launch_window_as<RT, 2, kMode, 64>(p, rows, stream);
     else
-      launch_window_blk<RT, kMode, 64>(p, rows, stream);
+      launch_window_as<RT, 2, kMode, 32>(p, rows, stream);
   } else {
-    launch_window_blk<RT, kMode, 64>(p, rows, stream);
+    launch_window_as<RT, 2, kMode, 64>(p, rows, stream);
   }
 }
 
 // Launches the window kernel over at most `rows` query rows.
 template <int kMode>
 void launch_window(const WindowParams& p, int64_t rows, hipStream_t stream) {
+  if (narrow_tasks<kMode>(p, rows)) return launch_window_as<1, 1, kMode, 32>(p, rows, stream);
   switch (row_tiles(p.Hq / p.Hkv)) {
-    case 1: return launch_window_rt<1, kMode>(p, rows, stream);
-    case 2: return launch_window_rt<2, kMode>(p, rows, stream);
-    case 4: return launch_window_rt<4, kMode>(p, rows, stream);
-    default: return launch_window_rt<8, kMode>(p, rows, stream);
+    case 1: return launch_window_wide<1, kMode>(p, rows, stream);
+    case 2: return launch_window_wide<2, kMode>(p, rows, stream);
+    case 4: return launch_window_wide<4, kMode>(p, rows, stream);
+    default: return launch_window_wide<8, kMode>(p, rows, stream);
   }
 }
 

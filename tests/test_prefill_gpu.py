@@ -666,7 +666,15 @@ def test_window_attention_split_with_overlapping_queries(rect_ext, hq, hkv, last
     torch.cuda.synchronize()
     uo, ul = _unsplit(d, -1, case.sm_scale, qo=qo, kv=kv)
     own = slice(shared, last)  # (the shared rows are written by requests of two lengths, in no order)
-    assert torch.equal(out[own].view(torch.int16), uo[own].view(torch.int16)) and torch.equal(lse[own], ul[own])
+    if (hq, hkv) == (32, 4):  # the unsplit call's tasks are of the same shape
+        assert torch.equal(out[own].view(torch.int16), uo[own].view(torch.int16)) and torch.equal(lse[own], ul[own])
+    else:
+        # narrow tasks move the softmax reference point at other blocks, so
+        # each key's weight is rounded to bf16 (2^-9 at most, 2^-9 / sqrt(3)
+        # rms) at another scale, and the two results once more: 2 / sqrt(3) *
+        # 2^-9 of the row's norm in all; the lse sums are fp32 (20000 terms)
+        assert rel_l2(bits(_host_bits(out[own])), bits(_host_bits(uo[own]))) < 2 ** -8
+        np.testing.assert_allclose(lse[own].cpu().numpy(), ul[own].cpu().numpy(), atol=2e-5, rtol=1e-6)
     assert not (lse == 7.0).any()
 
 
@@ -689,11 +697,69 @@ def test_window_attention_split_keeps_infinities(rect_ext):
     assert torch.isfinite(out[4:][:, finite.to(out.device)]).all()
 
 
+# Ragged batches whose tasks take every shape of the plain form (at 256 CUs):
+# (hq, hkv, requests, rows, keys past the rows, window)
+WINDOW_SHAPES = [
+    # narrow: at most a task per CU; a few rows at any batch
+    (8, 1, 4, (1, 40), (0, 200), -1), (6, 2, 7, (14, 34), (0, 90), 40), (4, 1, 300, (1, 16), (0, 60), -1),
+    (2, 2, 300, (1, 16), (0, 60), 15),
+    # wide, 16-row blocks of 64 keys, several per request or one each; and of 32
+    (16, 2, 40, (90, 130), (0, 80), -1), (10, 2, 70, (100, 130), (0, 60), 100), (8, 1, 200, (1, 16), (0, 300), -1),
+    (8, 1, 300, (1, 16), (0, 300), -1), (14, 2, 60, (30, 49), (0, 300), 255), (24, 2, 40, (30, 49), (0, 100), 64),
+    # wide, 32, 64 and 128 rows, the last ones of a block, of a tile, of one row
+    (8, 2, 60, (62, 98), (0, 70), -1), (6, 2, 60, (30, 66), (0, 70), 33), (4, 2, 40, (100, 130), (0, 70), -1),
+    (4, 2, 40, (125, 131), (0, 70), 90), (3, 3, 40, (100, 130), (0, 70), -1), (2, 2, 20, (250, 258), (0, 70), 200),
+    # request offsets past the room beside two 64-key tiles per CU
+    (8, 1, 1100, (1, 40), (0, 30), -1),
+]
+
+
+@pytest.mark.parametrize("hq,hkv,batch,rows,past,window_left", WINDOW_SHAPES)
+def test_window_attention_task_shapes(rect_ext, hq, hkv, batch, rows, past, window_left):
+    """Every shape of task and key block, with ragged edges, against the oracle."""
+    print(f"task shapes: {hq}/{hkv} x {batch} rows {rows} window {window_left}", flush=True)
+    rng = np.random.default_rng(hq * 1000 + batch)
+    qo = rng.integers(rows[0], rows[1] + 1, batch)
+    qo[:2] = rows
+    kv = qo + rng.integers(past[0], past[1] + 1, batch)
+    case = syn.prefill_case(qo_lens=qo, kv_lens=kv, hq=hq, hkv=hkv, seed=900 + batch)
+    d = _dev_case(case)
+    out, lse = rect_ext.window_attention_return_lse(d["q"], d["k"], d["v"], d["qo"], d["kv"], d["idx"], window_left,
+                                                    case.sm_scale)
+    torch.cuda.synchronize()
+    eo, el = orc.window_attention(_bf(case.q), _bf(case.k), _bf(case.v), case.qo_indptr, case.kv_indptr,
+                                  case.kv_indices, window_left=window_left, sm_scale=case.sm_scale)
+    got, exp = bits(_host_bits(out)), bits(eo)
+    err = np.linalg.norm((got - exp).reshape(got.shape[0], -1), axis=1) / np.linalg.norm(exp.reshape(got.shape[0], -1), axis=1)
+    assert err.max() < 1e-2, int(err.argmax())
+    np.testing.assert_allclose(lse.cpu().numpy(), el, atol=2e-4, rtol=1e-5)
+
+
+@pytest.mark.parametrize("hq,hkv,batch,rows,M", [
+    (8, 2, 9, (1, 50), 17),      # narrow
+    (12, 2, 150, (10, 33), 32),  # wide, 16 rows x 8 heads
+    (8, 2, 150, (40, 70), 48),   # wide, 32 rows x 4 heads, the second block half full
+    (6, 2, 150, (40, 70), 33),   # and of one row
+    (4, 2, 130, (70, 90), 80),   # wide, 64 rows x 2 heads
+    (2, 2, 130, (120, 140), 130),  # wide, 128 rows
+])
+@pytest.mark.parametrize("F,sink_mode", [(0, 0), (40, 1)])
+def test_rectify_task_shapes(rect_ext, hq, hkv, batch, rows, M, F, sink_mode):
+    """Every task shape of the fused form against the oracle."""
+    print(f"rectify task shapes: {hq}/{hkv} x {batch} rows {rows} M={M} F={F}", flush=True)
+    rng = np.random.default_rng(hq * 1000 + batch)
+    qo = rng.integers(rows[0], rows[1] + 1, batch)
+    case = syn.prefill_case(qo_lens=qo, kv_lens=qo + rng.integers(0, 120, batch), hq=hq, hkv=hkv, seed=950 + batch)
+    e, g, _ = _run_rectify(rect_ext, case, S=64, F=F, sink_mode=sink_mode, M=M, R=batch,
+                           req_ids=rng.permutation(batch).tolist(), request_length=rng.integers(0, 90, batch).tolist(),
+                           q_post_cache=True, seed=batch)
+    _compare_ring(e, g, f"task shapes {hq}/{hkv}")
+
+
 @pytest.mark.parametrize("window_left", [0, 40, 255])
 def test_window_attention_over_a_far_pool(rect_ext, window_left):
-    """Windows of GQA-8 groups over a K/V set larger than the caches take
-    32-key blocks that skip key groups past a window's end: the same rows
-    against the oracle, with the entries named as part of a larger index."""
+    """32-key blocks, which skip key groups past a window's end, with the
+    entries named as part of an index that is far longer than the pool."""
     case = syn.prefill_case(qo_lens=[1, 17, 300, 64], kv_lens=[1, 40, 700, 64], hq=16, hkv=2, seed=81)
     d = _dev_case(case)
     idx = torch.zeros((1 << 28) // 1024 + 1, dtype=torch.int32, device="cuda")  # more than 256 MiB of K/V rows
