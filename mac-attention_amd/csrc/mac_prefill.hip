@@ -1001,15 +1001,19 @@ __global__ void __launch_bounds__(256) window_combine_kernel(WindowParams p) {
     lt *= keep;
     o[0] *= keep;
     o[1] *= keep;
-#pragma unroll
-    for (int u = 0; u < kBatch; ++u) {
-      // (past the last piece: nothing, not its copy with weight 0, which may hold infinities)
-      const bool in = c0 + u < n;
-      const float f = in ? fast_exp2(w[u] - mx) : 0.0f;
-      const f32x4_t zero = {0.0f, 0.0f, 0.0f, 0.0f};
+    auto add = [&](int u) {
+      const float f = fast_exp2(w[u] - mx);
       lt += f * l[u];
-      o[0] += f * (in ? a[u][0] : zero);
-      o[1] += f * (in ? a[u][1] : zero);
+      o[0] += f * a[u][0];
+      o[1] += f * a[u][1];
+    };
+    if (c0 + kBatch <= n) {
+#pragma unroll
+      for (int u = 0; u < kBatch; ++u) add(u);
+    } else {  // (uniform) not the copies of the last piece, whose infinities a weight of 0 would keep
+#pragma unroll
+      for (int u = 0; u < kBatch; ++u)
+        if (c0 + u < n) add(u);
     }
   }
   const float inv = lt > 0.0f ? 1.0f / lt : 0.0f;
