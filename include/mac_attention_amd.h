@@ -282,8 +282,9 @@ MAC_API int mac_prefill_window_attention_bf16(const MacWindowAttentionArgs* args
  * until the call's work on `stream` is done), which lets a batch of few query
  * rows over many keys (no window) split its keys over the GPU; results differ
  * from the call without one by rounding only.  Without the bytes that
- * mac_prefill_window_attention_workspace names -- 0: the shape gains nothing
- * from a split -- the call runs unsplit.  No reference counterpart. */
+ * mac_prefill_window_attention_workspace names -- 0: no split for the shape --
+ * the call runs unsplit, and it may with them, where a split would cost more
+ * than it gains.  No reference counterpart. */
 MAC_API int mac_prefill_window_attention_ws_bf16(const MacWindowAttentionArgs* args, void* workspace,
                                                  int64_t workspace_bytes, void* stream);
 MAC_API int64_t mac_prefill_window_attention_workspace(int32_t B, int32_t Hq, int32_t Hkv, int64_t total_q,

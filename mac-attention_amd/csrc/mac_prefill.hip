@@ -1093,9 +1093,7 @@ int64_t expected_tasks(int64_t rows, int B, int Hq, int Hkv, int rt, int heads) 
 // one), three 328, 194 and 167 (a piece's state is 64 KiB written and read
 // once), half a round 430 for the first.  From
 // 3/4 of a round of tasks on the cut costs what it levels out (32 requests x
-// 32 rows over 4K keys, 8 heads per group: 129 unsplit, 141 split), and below
-// kSplitKeys keys per request the second launch does (512 rows over 1024
-// keys: 34 and 36; 32 rows over 1024 keys: 33 and 25).
+// 32 rows over 4K keys, 8 heads per group: 129 unsplit, 141 split).
 constexpr int64_t kSplitKeys = 1024;
 struct Split {
   int64_t blocks = 0;  // bound on the batch's row blocks
@@ -1119,6 +1117,23 @@ Split split_plan(int B, int Hq, int Hkv, int64_t total_q, int64_t kv_len, int wi
   sp.o_bytes = static_cast<size_t>(pieces * per_piece) * kTiles * 8 * 64 * 16;
   sp.bytes = sp.o_bytes + static_cast<size_t>(pieces * per_piece) * kTiles * 16 * 2 * sizeof(float);
   return sp;
+}
+
+// Whether a call that split_plan allows is cut: the states and the second
+// launch cost it 10-30 us, the more the more tasks it has (each in up to 5
+// pieces already at 1024 keys), and what it saves is the part of a task's
+// chain that idle CUs take over.  Keys per request from which it gains, in us
+// unsplit / split (1-row requests over 4 or 8 KV heads): 96 tasks, 1100 keys
+// 30.8 / 29.3; 128, 1100 keys 30 / 35, 1500 38 / 36; 160, 2000 keys 48 / 52, 3000
+// 70 / 67; 192, 3000 keys 88 / 92, 4000 129 / 123; 256, 3000 keys 109 / 112, 4000
+// 141 / 141, 8000 277 / 246; 1000 rows of one request (252), 3000 keys 84 / 86, 4000
+// 110 / 104.
+bool split_pays(const WindowParams& p) {
+  const int64_t cus = device_cus();
+  const int rt = row_tiles(p.Hq / p.Hkv);
+  const int64_t tasks = expected_tasks(p.total_q, p.B, p.Hq, p.Hkv, rt, kTiles / rt);
+  const int64_t line = (tasks - 68 * cus / 256) * 6400 / cus;  // 25 keys per task past 68 of 256 CUs
+  return p.kv_len_total / p.B >= (tasks <= cus ? std::min<int64_t>(line, 4000) : line);
 }
 
 template <int RT>
@@ -1330,7 +1345,7 @@ extern "C" int mac_prefill_window_attention_ws_bf16(const MacWindowAttentionArgs
   const Split sp = workspace != nullptr
                        ? split_plan(a->B, a->Hq, a->Hkv, a->total_q, a->kv_indices_len, a->window_left)
                        : Split{};
-  if (sp.pieces > 0 && static_cast<int64_t>(sp.bytes) <= workspace_bytes) {
+  if (sp.pieces > 0 && static_cast<int64_t>(sp.bytes) <= workspace_bytes && split_pays(p)) {
     p.part_o = static_cast<float*>(workspace);
     p.part_ml = reinterpret_cast<float*>(static_cast<char*>(workspace) + sp.o_bytes);
     p.max_pieces = sp.pieces;

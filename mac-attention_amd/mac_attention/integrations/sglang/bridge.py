@@ -804,8 +804,8 @@ class PrefillRectifyExtension:
             # few rows over many keys: room for the partial states of a split
             # over keys, from PyTorch's allocator (its stream-ordered reuse
             # and graph pools keep it safe across streams and captures)
-            n = self._lib.mac_prefill_window_attention_workspace(a.B, a.Hq, a.Hkv, total_q, a.kv_indices_len,
-                                                                 a.window_left)
+            n = 0 if a.window_left >= 0 else self._lib.mac_prefill_window_attention_workspace(
+                a.B, a.Hq, a.Hkv, total_q, a.kv_indices_len, a.window_left)
             ws = torch.empty(n, device=q.device, dtype=torch.uint8) if n > 0 else None
             rc = self._lib.mac_prefill_window_attention_ws_bf16(ctypes.byref(a), _ptr(ws), n, _stream(q.device))
         _raise_on(self._lib, rc)

@@ -678,6 +678,18 @@ def test_window_attention_split_with_overlapping_queries(rect_ext, hq, hkv, last
     assert not (lse == 7.0).any()
 
 
+@pytest.mark.parametrize("batch,rows,kv", [(64, 1, 1100), (1, 1000, 1100), (24, 17, 1030)])
+def test_window_attention_split_where_it_pays(rect_ext, batch, rows, kv):
+    """Calls with a task for most CUs and few keys are not cut, workspace or
+    not: the bits of the call without one."""
+    case = syn.prefill_case(qo_lens=[rows] * batch, kv_lens=[kv] * batch, hq=32, hkv=4, seed=72)
+    d = _dev_case(case)
+    assert _workspace_bytes(d) > 0
+    out, lse = rect_ext.window_attention_return_lse(d["q"], d["k"], d["v"], d["qo"], d["kv"], d["idx"], -1, case.sm_scale)
+    uo, ul = _unsplit(d, -1, case.sm_scale)
+    assert torch.equal(out.view(torch.int16), uo.view(torch.int16)) and torch.equal(lse, ul)
+
+
 def test_window_attention_split_keeps_infinities(rect_ext):
     """A row's infinite value stays infinite, in whichever of its pieces the
     key falls, and touches no other dim: the combining kernel adds no piece
