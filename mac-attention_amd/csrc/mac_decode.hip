@@ -2501,7 +2501,7 @@ int mac::decode_impl(const MacDecodeArgs* a, void* stream_ptr, hipEvent_t* ev) {
   MAC_REQUIRE(a->tile_tokens > 0 && a->match_tile_slots > 0, "tile sizes must be positive");
   MAC_REQUIRE(a->max_match_tiles >= (M + a->match_tile_slots - 1) / a->match_tile_slots && a->max_match_tiles > 0,
               "match workspace too small");
-  MAC_REQUIRE(a->max_tiles_context >= (a->max_context + a->tile_tokens - 1) / a->tile_tokens,
+  MAC_REQUIRE(a->max_tiles_context >= (static_cast<int64_t>(a->max_context) + a->tile_tokens - 1) / a->tile_tokens,
               "rect workspace too small");
   MAC_REQUIRE(a->max_tiles_context >= 4,
               "rect workspace too small: this build needs at least 4 partial slots per group");

@@ -139,7 +139,7 @@ extern "C" int mac_persistent_decode_bf16_noalloc(const MacDecodeArgs* a, void* 
   w.match_tile_slots = 256;
   const int slots = kPartialSlots * share;
   w.max_tiles_context = slots;
-  w.tile_tokens = (a->max_context + slots - 1) / slots;
+  w.tile_tokens = static_cast<int32_t>((static_cast<int64_t>(a->max_context) + slots - 1) / slots);
   w.complete_task_len = 2 * static_cast<int64_t>(a->N) * (a->Hkv > 0 ? a->Hkv : 1) + kTaskExtra;
   w.workspace_rows = a->N;
   rc = mac_persistent_decode_bf16(&w, stream_ptr);

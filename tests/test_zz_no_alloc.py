@@ -141,6 +141,20 @@ def test_noalloc_entry_at_a_2048_slot_ring_and_128k_context(ext):
     _assert_same(runs["noalloc"], runs["workspace"], 1e-3)
 
 
+def test_noalloc_entry_takes_the_largest_max_context(ext):
+    """max_context only bounds the contexts: any positive value is taken."""
+    b, hq, hkv, kv_lens, m, s, f, hit_rate, seed = CASES[1]
+    c = syn.random_case(batch=b, hq=hq, hkv=hkv, kv_lens=kv_lens, capacity=m, semantic_pos_ahead=s,
+                        front_sink_tokens=f, hit_rate=hit_rate, match_lag=m // 2, seed=seed)
+    res = oracle_run(c)
+    dev = syn.to_device(torch, c)
+    out = torch.empty_like(dev["q_post"])
+    out_lse = torch.empty(b, hq, device="cuda")
+    ext.mac_persistent_decode_bf16_noalloc(*_args(dev, c, [None] * 30, out, out_lse, 2 ** 31 - 100))
+    torch.cuda.synchronize()
+    assert rel_l2(_np(out), bits(res.out)) < 1e-2
+
+
 def test_noalloc_entry_replays_from_a_graph(ext):
     """The no-allocation step captured in a hipGraph (the callers it is for):
     three replays, with the ring restored and eager work between them, each
