@@ -3,9 +3,10 @@ libmac_noalloc.so, workspaces in that library's static device array) against
 the ordinary entry point on the same inputs, through the C ABI: two calls in
 a row, the second with a smaller step, each compared output for output (and
 with the oracle); the workspace arguments may be None; a ring of 2048 slots
-(the range-split scan) at a context near 128K (chunks enlarged to fit the
-array's 32 partial slots per group); replays of a captured graph; and the
-size limits are refused with a clear error."""
+(the range-split scan) at a context near 128K; a step of so many heads that
+its long groups' chunks are enlarged to fit the array's 32 partial slots per
+group; the largest max_context; replays of a captured graph; and the size
+limits are refused with a clear error."""
 
 import numpy as np
 import pytest
@@ -115,9 +116,9 @@ def _big_case():
 
 
 def test_noalloc_entry_at_a_2048_slot_ring_and_128k_context(ext):
-    """The range-split ring scan and a 127K-token context, where the array's
-    32 partial slots per group make the plan enlarge the long groups' chunks
-    (so the sums differ from the workspace entry's only by rounding)."""
+    """The range-split ring scan and a 127K-token context.  The step's 64
+    heads have 2048 of the array's partial slots per group, so its chunks are
+    the workspace entry's; the sums may differ from it by rounding only."""
     dev, b, hq, hkv, m, S = _big_case()
     pristine = {k: dev[k].clone() for k in ("query_cache", "attn_cache", "lse_cache")}
     max_context = 131072
@@ -139,6 +140,36 @@ def test_noalloc_entry_at_a_2048_slot_ring_and_128k_context(ext):
         runs[mode] = _state(dev, out, out_lse)
     assert hits == round(0.8 * b * hq)
     _assert_same(runs["noalloc"], runs["workspace"], 1e-3)
+
+
+def test_noalloc_entry_enlarges_chunks_for_many_heads(ext):
+    """2080 query heads leave each group 32 partial slots; the four groups of
+    the one long context would have about 125 chunks of 1024 tokens (520K
+    tokens over 512 workgroups), which are enlarged to fit."""
+    b, hq, hkv, S = 65, 32, 4, 64
+    kv_lens = [127000] + [90 + 3 * i for i in range(b - 1)]
+    c = syn.random_case(batch=b, hq=hq, hkv=hkv, kv_lens=kv_lens, capacity=16, semantic_pos_ahead=S, front_sink_tokens=8,
+                        hit_rate=0.0, seed=75)
+    res = oracle_run(c)
+    max_context = 131072
+    dev = syn.to_device(torch, c)
+    out = torch.empty_like(dev["q_post"])
+    out_lse = torch.empty(b, hq, device="cuda")
+    print("no-alloc 2080 heads, one context of 127000", flush=True)
+    ext.mac_persistent_decode_bf16_noalloc(*_args(dev, c, [None] * 30, out, out_lse, max_context))
+    torch.cuda.synchronize()
+    n = _state(dev, out, out_lse)
+    assert rel_l2(n["out"], bits(res.out)) < 1e-2
+    assert rel_l2(n["out"][0], bits(res.out)[0]) < 1e-2  # the long context by itself
+    np.testing.assert_array_equal(n["q"], res.query_cache)
+    assert rel_l2(n["a"], bits(res.attn_cache)) < 1e-2
+    # the workspace entry cuts the same groups into more pieces: the sums differ by rounding only
+    dev = syn.to_device(torch, c)
+    out2, out_lse2, ws = syn.run_decode(torch, ext, dev, c, max_context=max_context, tile_tokens=32, match_tile_slots=32)
+    torch.cuda.synchronize()
+    tasks = _np(ws[17]).reshape(-1)[:hkv]  # complete_task_tile: the tasks of the first request's groups
+    assert tasks.max() > 32, tasks
+    _assert_same(n, _state(dev, out2, out_lse2), 1e-3)
 
 
 def test_noalloc_entry_takes_the_largest_max_context(ext):
