@@ -447,19 +447,29 @@ __global__ void __launch_bounds__(256, (kPer == 1 && kMode == kPlain) ? 3 : 2) w
   //    eighths as above (2-3% faster than round-robin; head-major was slower);
   //  * causal (window_left < 0) and split: row-block order dealt
   //    round-robin.  Causal tasks grow with the row block, and a workgroup
-  //    keeps its offset within every round, so a head-major order would give
-  //    some workgroups only the longest tasks.
+  //    would keep its offset within every round: with as many tasks per request
+  //    as divide the grid (or nearly) some would take only the longest ones.
+  //    So every other round is dealt backwards (unsplit form: 8 x 1024 rows, 4
+  //    heads per group, 168 us forwards, 111 back and forth; 2 x 2048 rows 139
+  //    and 96), and so is a last, partial one (5 x 1037 rows 113 and 93); in
+  //    whole eights, so that an XCD keeps its KV heads.
   const int grid = gridDim.x;
   const int eighth = grid / 8;
   const int npieces = s_boff[B];
   const bool head_major = kMode == kPlain && wl >= 0;
   const bool by_xcd = (kFused || (kMode == kPlain && wl >= 0)) && grid % 8 == 0;
+  const bool back_and_forth = kMode == kPlain && wl < 0;
+  bool odd_round = true;
   for (int task = blockIdx.x; task < total_tasks; task += grid) {
     __syncthreads();  // the previous task's waves are done with the tiles
     const int round0 = task - static_cast<int>(blockIdx.x);
+    odd_round = !odd_round;
+    const int back = back_and_forth && (odd_round || (round0 > 0 && round0 + grid > total_tasks))
+                         ? min(grid, total_tasks - round0) & ~7  // tasks of the round dealt backwards
+                         : 0;
     const int t = (by_xcd && round0 + grid <= total_tasks)
                       ? round0 + (static_cast<int>(blockIdx.x) % 8) * eighth + static_cast<int>(blockIdx.x) / 8
-                      : task;
+                      : (static_cast<int>(blockIdx.x) < back ? task + back - 8 - 2 * (static_cast<int>(blockIdx.x) & ~7) : task);
     int piece, hc;  // piece; KV head * nchunks + head chunk
     if (head_major) {
       hc = t / npieces;
