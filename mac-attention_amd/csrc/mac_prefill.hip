@@ -1095,15 +1095,14 @@ int64_t expected_tasks(int64_t rows, int B, int Hq, int Hkv, int rt, int heads) 
 // keys in one chain, so a batch with few of them leaves CUs idle; its keys
 // are then cut so that there are up to two rounds of the resident workgroups
 // (2 per CU) more tasks than row blocks.  Kept suffixes of long prompts are
-// that case: 512 rows over 32K keys, 4 heads per group, 839 -> 318 us
-// unsplit -> split; 8 requests of 16-32 rows over 8K-64K keys, 8 heads per
-// group, 1329 -> 196; one row over 127K keys 3340 -> 134.  One round more
-// instead took 318, 224 and 98 us (no second round to level the ragged
-// batch), 1.5 rounds 323, 196 and 115 (a half-empty last round for the even
-// one), three 328, 194 and 167 (a piece's state is 64 KiB written and read
-// once), half a round 430 for the first.  From
-// 3/4 of a round of tasks on the cut costs what it levels out (32 requests x
-// 32 rows over 4K keys, 8 heads per group: 129 unsplit, 141 split).
+// that case.  Unsplit, half a round, one, 1.5, two and three rounds of pieces
+// took (us): 512 rows over 32K keys, 4 heads per group, 681, 430, 317, 329, 322
+// and 331; 8 requests of 16-32 rows over 8K-64K keys, 8 heads per group, 1302,
+// 253, 231, 203, 187 and 199; one row over 127K keys, 4 KV heads, 2768, 84, 80,
+// 93, 104 and 124 (a piece's state is 64 KiB written and read once): one round
+// leaves a ragged batch nothing to level it with.  From 3/4 of a round of tasks
+// on the cut costs what it levels out (32 requests x 32 rows over 4K keys, 8
+// heads per group: 129 unsplit, 141 split).
 constexpr int64_t kSplitKeys = 1024;
 struct Split {
   int64_t blocks = 0;  // bound on the batch's row blocks
@@ -1203,21 +1202,23 @@ bool narrow_tasks(const WindowParams& p, int64_t rows) {
 // the GPU has more than a round of tasks; and for single blocks over whole
 // prefixes while it has at most one task per CU.  Elsewhere 32, whose window
 // ends nearer to what it loads and which waits for fewer keys at a time.  32
-// also for windows over a K/V set that the caches do not hold (the loads past a
-// window's end go to HBM) and for batches whose request offsets leave a CU no
-// room for two workgroups with 64.  Times in us, 64 / 32 (8 heads per group):
-// 30 x 100 rows over 1500 keys 125 / 129; 8 x 200 over 200, 17.7 / 18.9; 8 x
-// 8192, window 256, 553 / 558; 1 row over 3000 keys 81 / 86; 96 requests of 1
-// row over 1500 keys (384 tasks) 78 / 69; 500 x 16 rows over 300 keys 120 / 116;
-// 16 x 64 rows, window 256, 19.0 / 18.0; 1100 x 16 over 300 keys 287 / 231; 64
-// x 8192, window 256 (1.07 GB of K/V), 4640 / 4470.
-constexpr int64_t kFarBytes = 256ll << 20;  // the memory-side cache
+// also for windows of up to 64 keys, windows over a K/V set that the caches do
+// not hold (what is loaded past a window's end comes from HBM; counted as the
+// index entries, at most the pool's rows), and batches whose request offsets
+// leave a CU no room for two workgroups with 64.  Times in us, 64 / 32 (8 heads
+// per group): 30 x 100 rows over 1500 keys 125 / 129; 8 x 200 over 200, 17.7 /
+// 18.9; 1 row over 3000 keys 81 / 86; 96 requests of 1 row over 1500 keys (384
+// tasks) 78 / 69; 500 x 16 rows over 300 keys 120 / 116; 16 x 64 rows, window 256,
+// 19.0 / 18.0; 1100 x 16 over 300 keys 287 / 231.  N x 8192 rows, window 256, 16
+// MiB of K/V each: 12, 815 / 820; 24, 1637 / 1639; 32, 2178 / 2174; 48, 3341 /
+// 3285; 64, 4497 / 4367; window 64: 16, 729 / 709.
+constexpr int64_t kFarBytes = 512ll << 20;  // twice the memory-side cache
 
 bool long_blocks(const WindowParams& p, int64_t rows, size_t request_bytes) {
   const int64_t cus = device_cus();
   const int64_t tasks = expected_tasks(rows, p.B, p.Hq, p.Hkv, 1, kTiles);
   const int64_t far = std::min(p.kv_len_total, p.pool_tokens) * p.Hkv * (4 * kHeadDim);
-  if (p.window_left >= 0 && far > kFarBytes) return false;
+  if (p.window_left >= 0 && (p.window_left < 64 || far > kFarBytes)) return false;
   int per_cu = 0;
   const void* kern = reinterpret_cast<const void*>(&window_kernel<1, 2, kPlain, 64>);
   if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, 256, request_bytes) != hipSuccess || per_cu < 2) return false;
