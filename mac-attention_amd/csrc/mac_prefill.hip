@@ -451,8 +451,9 @@ __global__ void __launch_bounds__(256, (kPer == 1 && kMode == kPlain) ? 3 : 2) w
   //    as divide the grid (or nearly) some would take only the longest ones.
   //    So every other round is dealt backwards (unsplit form: 8 x 1024 rows, 4
   //    heads per group, 168 us forwards, 111 back and forth; 2 x 2048 rows 139
-  //    and 96), and so is a last, partial one (5 x 1037 rows 113 and 93); in
-  //    whole eights, so that an XCD keeps its KV heads.
+  //    and 96), and so is a last, partial one (5 x 1037 rows 113 and 93).
+  //    Backwards in whole eights, which keeps an XCD's KV heads, gained nothing
+  //    (8 heads per group and 4 KV heads, 5 x 1037 rows, 96 and 118).
   const int grid = gridDim.x;
   const int eighth = grid / 8;
   const int npieces = s_boff[B];
@@ -464,12 +465,10 @@ __global__ void __launch_bounds__(256, (kPer == 1 && kMode == kPlain) ? 3 : 2) w
     __syncthreads();  // the previous task's waves are done with the tiles
     const int round0 = task - static_cast<int>(blockIdx.x);
     odd_round = !odd_round;
-    const int back = back_and_forth && (odd_round || (round0 > 0 && round0 + grid > total_tasks))
-                         ? min(grid, total_tasks - round0) & ~7  // tasks of the round dealt backwards
-                         : 0;
+    const bool backwards = back_and_forth && (odd_round || (round0 > 0 && round0 + grid > total_tasks));
     const int t = (by_xcd && round0 + grid <= total_tasks)
                       ? round0 + (static_cast<int>(blockIdx.x) % 8) * eighth + static_cast<int>(blockIdx.x) / 8
-                      : (static_cast<int>(blockIdx.x) < back ? task + back - 8 - 2 * (static_cast<int>(blockIdx.x) & ~7) : task);
+                      : (backwards ? round0 + min(grid, total_tasks - round0) - 1 - static_cast<int>(blockIdx.x) : task);
     int piece, hc;  // piece; KV head * nchunks + head chunk
     if (head_major) {
       hc = t / npieces;
