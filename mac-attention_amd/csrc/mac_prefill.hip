@@ -449,17 +449,25 @@ __global__ void __launch_bounds__(256, (kPer == 1 && kMode == kPlain) ? 3 : 2) w
   //    round-robin.  Causal tasks grow with the row block, and a workgroup
   //    would keep its offset within every round: with as many tasks per request
   //    as divide the grid (or nearly) some would take only the longest ones.
-  //    So every other round is dealt backwards (unsplit form: 8 x 1024 rows, 4
+  //    So with as many row blocks in every request, where the offsets recur,
+  //    every other round is dealt backwards (unsplit form: 8 x 1024 rows, 4
   //    heads per group, 168 us forwards, 111 back and forth; 2 x 2048 rows 139
   //    and 96), and so is a last, partial one (5 x 1037 rows 113 and 93).
-  //    Backwards in whole eights, which keeps an XCD's KV heads, gained nothing
-  //    (8 heads per group and 4 KV heads, 5 x 1037 rows, 96 and 118).
+  //    Ragged batches only gain and lose by it (5 x 765-1529 rows, 8 heads per
+  //    group, 136 and 153).  Backwards in whole eights, which keeps an XCD's KV
+  //    heads, gained nothing (8 heads per group and 4 KV heads, 5 x 1037 rows,
+  //    96 and 118).
   const int grid = gridDim.x;
   const int eighth = grid / 8;
   const int npieces = s_boff[B];
   const bool head_major = kMode == kPlain && wl >= 0;
   const bool by_xcd = (kFused || (kMode == kPlain && wl >= 0)) && grid % 8 == 0;
-  const bool back_and_forth = kMode == kPlain && wl < 0;
+  bool back_and_forth = false;
+  if (kMode == kPlain && wl < 0) {
+    int same = 1;
+    for (int b = tid; b < B; b += 256) same &= s_boff[b + 1] - s_boff[b] == s_boff[1];
+    back_and_forth = __syncthreads_and(same) != 0;
+  }
   bool odd_round = true;
   for (int task = blockIdx.x; task < total_tasks; task += grid) {
     __syncthreads();  // the previous task's waves are done with the tiles
