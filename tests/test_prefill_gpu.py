@@ -721,8 +721,9 @@ WINDOW_SHAPES = [
     # wide, 32, 64 and 128 rows, the last ones of a block, of a tile, of one row
     (8, 2, 60, (62, 98), (0, 70), -1), (6, 2, 60, (30, 66), (0, 70), 33), (4, 2, 40, (100, 130), (0, 70), -1),
     (4, 2, 40, (125, 131), (0, 70), 90), (3, 3, 40, (100, 130), (0, 70), -1), (2, 2, 20, (250, 258), (0, 70), 200),
-    # more than two rounds of the grid, the last one partial
-    (8, 2, 400, (20, 60), (0, 40), -1), (4, 1, 1700, (1, 16), (0, 20), -1),
+    # more than two rounds of the grid, the last one partial: ragged, and as many row blocks in every request
+    (8, 2, 400, (20, 60), (0, 40), -1), (8, 2, 300, (60, 64), (0, 90), -1), (16, 2, 150, (65, 80), (0, 90), -1),
+    (4, 1, 1700, (1, 16), (0, 20), -1),
     # request offsets past the room beside two 64-key tiles per CU
     (8, 1, 1100, (1, 40), (0, 30), -1),
 ]
